@@ -96,7 +96,12 @@ typedef struct srt_tile_config {
     int b_staging;         /* B operand path: 1 = copy the workgroup's B tile (K rows x
                               N_c columns) into LDS once and read packed columns
                               from there; 2 = read B rows from global memory per
-                              packed column; 0 = choose (global memory)          */
+                              packed column; 3 = streamed (M_r = 1 mappings, whose
+                              chains run in column order): tiles of B rows staged in
+                              LDS one after another, chunk_cols (1, 2, 4, 8) C rows
+                              per wave, waves_per_block 4, 8 or 16, one chain per
+                              row (nsplit 1); 0 = choose (3 where it applies, else
+                              global memory)                                      */
     int layout;            /* wave slots -> workgroups: 1 = panels in order, a panel
                               on kp waves as chunk_cols says; 2 = balanced: panels
                               binned heaviest-first into the least-loaded of G

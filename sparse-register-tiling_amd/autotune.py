@@ -439,15 +439,60 @@ def add_candidate(cache: "TuningCache", case, mapping: Tuple[int, str], shape: D
     return rec
 
 
+# Streamed execution (one row per panel, B tiles in LDS) against the gather
+# executor, for sizes the table does not hold.  Fitted to 90 sizes (M 512-4096,
+# K 512-4096, sparsity 0.70-0.95, N 128-2048; 256 CUs, 2.4 GHz).  Per lane
+# width V: clocks of a workgroup's B tile when staging bounds it, clocks per
+# entry, clocks per tile beside the entries.
+STREAM_COST = {1: (7000.0, 2.8, 4000.0), 2: (5600.0, 4.7, 2500.0), 4: (4800.0, 8.5, 2000.0)}
+STREAM_WAVES = 16
+
+
+def streamed_launch(M: int, K: int, nnz: int, N: int) -> Tuple[int, int, float]:
+    """(lane width, rows per wave, estimated seconds) of the fastest streamed
+    launch.  A wide lane halves the LDS reads per product, a narrow one the
+    B bytes a workgroup stages; rows per wave fill the chip's 256 workgroups
+    once (a second round costs a whole pass).  A row's entries of a tile are
+    padded to four: 1.5 more on average."""
+    best = (1, 1, float("inf"))
+    for V, (staging, per_entry, per_tile) in STREAM_COST.items():
+        rows = 16 * STREAM_WAVES // V  # B rows of a tile
+        tiles = -(-max(K, 1) // rows)
+        for R in (1, 2, 4, 8):
+            groups = -(-M // (STREAM_WAVES * R)) * -(-max(N, 1) // (64 * V))
+            entries = STREAM_WAVES * R * (nnz / float(max(1, M * tiles)) + 1.5)
+            tile = max(staging, per_entry * entries + per_tile)
+            t = 2.2e-6 + -(-groups // 256) * tiles * tile / 2.4e9
+            if t < best[2]:
+                best = (V, R, t)
+    return best
+
+
+def gather_seconds(M: int, K: int, nnz: int, N: int) -> float:
+    """Estimated seconds of the gather executor with the 4-row "orig" mapping
+    on the same sizes: 4 us and 0.16 us per 10^6 products, times the packed
+    columns per nonzero of a 4-row panel (one B row gathered for each)."""
+    d = nnz / float(max(1, M * K))
+    share = (1.0 - (1.0 - d) ** 4) / (4.0 * d) if d > 0 else 1.0
+    return 4e-6 + 0.16e-12 * share * nnz * N
+
+
 def tuned_plan(csr: torch.Tensor, N: int, path: str = SHIPPED) -> MatMulSpecialized:
     """A plan with the best measured configuration of the tuning table for
     this shape, sparsity bucket and N (the reference's heuristic-JSON lookup,
-    tools/paper/heuristic.py:26-50, experiment_runner.py:86-113); the default
-    configuration when the table has no entry."""
+    tools/paper/heuristic.py:26-50, experiment_runner.py:86-113).  Where the
+    table has no entry: streamed execution when its estimate is the lower
+    one, else the default configuration."""
     M, K = csr.shape
     sparsity = 1.0 - csr.values().numel() / float(max(1, M * K))
     recs = TuningCache(path).get(M, K, sparsity, N)
     if not recs:
+        nnz = csr.values().numel()
+        V, R, seconds = streamed_launch(M, K, nnz, N)
+        if seconds < gather_seconds(M, K, nnz, N):
+            return MatMulSpecialized.from_csr(csr, N, mapping_id=named_mapping(1, "identity"),
+                                              tile_config=TileConfig(b_staging=3, vec_width=V, waves_per_block=16,
+                                                                     chunk_cols=R))
         return MatMulSpecialized.from_csr(csr, N, mapping_id=named_mapping(4, "orig"))
     (M_r, name), cfg = best_config(recs)
     return MatMulSpecialized.from_csr(csr, N, mapping_id=named_mapping(M_r, name), tile_config=cfg)

@@ -40,7 +40,7 @@ CFLAGS = [
     "-I" + INCLUDE, "-I" + CSRC,
 ]
 HAND_SOURCES = ["capi.hip", "packer.hip", "csr_spmm.hip", "mfma_panel.hip", "mfma_capi.hip", "probe.hip", "dense_panels.hip",
-                "mfma_exec.hip"]
+                "mfma_exec.hip", "stream_exec.hip"]
 
 
 def _load_sibling(name):

@@ -387,6 +387,11 @@ struct srt_plan {
     int device = 0;
     std::vector<RetiredSchedule> retired;  // schedules of earlier widths, alive until destroy
     DensePart dense;                       // hybrid plans: panels on matrix cores
+    // b_staging 3: the streamed schedule (retired ones stay alive for graphs
+    // that captured them); sch is then built only when something asks for it
+    StreamSched stream;
+    std::vector<StreamSched> retired_streams;
+    std::mutex mu;
     // matrix_cores: panel ranges for R ranges (the last entry is current;
     // earlier ones stay alive for graphs that captured them)
     std::vector<std::pair<int, int32_t *>> mfma_ranges;
@@ -625,6 +630,38 @@ static void realise_config(srt_tile_config &c, int M_r, int K, int K_tile, int64
     c.K_c = K_tile;
 }
 
+// Streamed execution: the packing's chains run in column order.
+static bool column_ordered(const ExecutorDesc *e) { return e->M_r == 1 && e->num_patterns == 1; }
+
+static bool streamed(const srt_tile_config &c) { return c.b_staging == 3; }
+
+// Realise the streamed launch of an M x K matrix at width n: lane width V,
+// waves per workgroup W, C rows per wave R (chunk_cols).
+static void realise_stream(srt_tile_config &c, int M, int K, int K_tile, int64_t nnz, int n) {
+    if (c.waves_per_block != 4 && c.waves_per_block != 8 && c.waves_per_block != 16) c.waves_per_block = 16;
+    // One workgroup per CU in one round takes V * R = M n / (64 * waves of the
+    // chip); wide lanes read the LDS best, so V grows with the work first,
+    // then R (measured: 4 x 8 down to 2 x 2 lead at every size tried).
+    const int64_t vr = std::max<int64_t>(1, (int64_t)M * n / (64 * (int64_t)cu_count() * c.waves_per_block));
+    if (c.vec_width != 1 && c.vec_width != 2 && c.vec_width != 4)
+        c.vec_width = vr >= 16 && n > 128 ? 4 : vr >= 2 && n > 64 ? 2 : 1;
+    if (c.chunk_cols != 1 && c.chunk_cols != 2 && c.chunk_cols != 4 && c.chunk_cols != 8) {
+        const int64_t slices = (n + 64 * c.vec_width - 1) / (64 * c.vec_width);
+        const int64_t waves = (int64_t)cu_count() * c.waves_per_block;
+        const int64_t rows = ((int64_t)M * slices + waves - 1) / waves;
+        c.chunk_cols = rows <= 1 ? 1 : rows <= 2 ? 2 : rows <= 4 ? 4 : 8;
+    }
+    if (c.xcd_remap != 0 && c.xcd_remap != 1) c.xcd_remap = 1;
+    if (!pow2_upto8(c.unroll)) c.unroll = 4;
+    if (c.layout != 1 && c.layout != 2) c.layout = 2;
+    c.b_staging = 3;
+    c.nsplit = 1;
+    c.matrix_cores = 0;
+    c.M_c = c.waves_per_block * c.chunk_cols;
+    c.N_c = 64 * c.vec_width;
+    c.K_c = K_tile;
+}
+
 static bool aligned(const void *p, int bytes) { return ((uintptr_t)p % (uintptr_t)bytes) == 0; }
 
 static int run_executor(const Packed &pk, const Schedule &sch, const ExecutorDesc *exec,
@@ -687,6 +724,21 @@ static int run_executor(const Packed &pk, const Schedule &sch, const ExecutorDes
     a.xcd_remap = cfg.xcd_remap;
     a.unroll = sch.unroll;
     SRT_HIP_TRY(fn(a, s));
+    return SRT_OK;
+}
+
+static int run_stream(const Packed &pk, const StreamSched &st, const srt_tile_config &cfg, const float *B, int64_t ldb,
+                      float *C, int64_t ldc, int n, hipStream_t s) {
+    if (n < 0) return fail(SRT_ERR_INVALID, "n must be >= 0");
+    if (n == 0) return SRT_OK;
+    if (!B || !C) return fail(SRT_ERR_INVALID, "null B or C");
+    if (ldb < n || ldc < n) return fail(SRT_ERR_INVALID, "ldb and ldc must be >= n");
+    // B rows are addressed with a 32-bit byte offset (buffer loads).
+    if ((int64_t)pk.K * ldb * (int64_t)sizeof(float) > (int64_t)0xffffffffLL)
+        return fail(SRT_ERR_UNSUPPORTED, "B larger than 4 GiB (K * ldb * 4 bytes)");
+    StreamLaunch a{st.blocks, st.first, st.rows_of, B, C, ldb, ldc, n, pk.K, st.V, st.R, st.waves, st.n_wg,
+                   cfg.xcd_remap};
+    SRT_HIP_TRY(launch_stream(a, s));
     return SRT_OK;
 }
 
@@ -1008,6 +1060,73 @@ static int switch_schedule(const Packed &pk, const srt_tile_config &c, int tiles
     return SRT_OK;
 }
 
+void StreamSched::release() {
+    hipFree(blocks);
+    hipFree(first);
+    hipFree(rows_of);
+    blocks = first = nullptr;
+    rows_of = nullptr;
+}
+
+// Entry blocks of the streamed launch of config c: rows in order of falling
+// nonzeros are dealt to the waves boustrophedon (waves of all workgroups
+// first), so waves, workgroups and SIMDs get even shares; the blocks are
+// counted and written on the device.
+static int build_stream(const Packed &pk, const srt_tile_config &c, StreamSched &out, hipStream_t s) {
+    StreamSched st;
+    st.V = c.vec_width;
+    st.waves = c.waves_per_block;
+    st.R = c.chunk_cols;
+    std::vector<int> order;
+    order.reserve((size_t)pk.M);
+    for (int i = 0; i < pk.M; ++i)
+        if (pk.h_skip.empty() || !pk.h_skip[i]) order.push_back(i);
+    const int M = (int)order.size();
+    st.n_wg = std::max(1, (M + st.waves * st.R - 1) / (st.waves * st.R));
+    const int nw = st.n_wg * st.waves;
+    const int T = stream_tile_rows(st.V, st.waves), KT = (pk.K + T - 1) / T, BW = stream_block_words(st.V);
+    auto len = [&](int r) { return pk.h_col_ptr[r + 1] - pk.h_col_ptr[r]; };
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return len(a) > len(b); });
+    std::vector<int32_t> rows((size_t)nw * st.R, -1);
+    for (int i = 0; i < M; ++i) {
+        const int turn = i / nw, j = turn & 1 ? nw - 1 - i % nw : i % nw;
+        rows[((size_t)(j % st.n_wg) * st.waves + j / st.n_wg) * st.R + turn] = order[i];
+    }
+    Scratch sc;
+    int32_t *d_blk = nullptr;
+    SRT_TRY(sc.get(&d_blk, (size_t)nw * KT));
+    struct Guard {  // frees what a failure leaves behind
+        StreamSched *p;
+        ~Guard() { if (p) p->release(); }
+    } guard{&st};
+    SRT_TRY(dmalloc(&st.rows_of, rows.size()));
+    SRT_TRY(dmalloc(&st.first, (size_t)nw));
+    SRT_HIP_TRY(hipMemcpyAsync(st.rows_of, rows.data(), sizeof(int32_t) * rows.size(), hipMemcpyHostToDevice, s));
+    SRT_HIP_TRY(launch_stream_count(nw, st.R, st.V, st.waves, pk.K, st.rows_of, pk.col_ptr, pk.cols, d_blk, st.first, s));
+    std::vector<uint32_t> first((size_t)nw);
+    SRT_HIP_TRY(hipMemcpyAsync(first.data(), st.first, sizeof(uint32_t) * nw, hipMemcpyDeviceToHost, s));
+    SRT_HIP_TRY(hipStreamSynchronize(s));
+    uint64_t total = 0;
+    for (uint32_t &f : first) {
+        const uint32_t n = f;
+        f = (uint32_t)total;
+        total += n;
+    }
+    // The executor loads up to three blocks past a wave's last one.
+    const size_t words = (size_t)(total + 3) * BW;
+    if (words > 0xffffffffULL) return fail(SRT_ERR_UNSUPPORTED, "streamed entries exceed 16 GiB");
+    SRT_TRY(dmalloc(&st.blocks, words));
+    SRT_HIP_TRY(hipMemsetAsync(st.blocks + (size_t)total * BW, 0, sizeof(uint32_t) * 3 * BW, s));
+    SRT_HIP_TRY(hipMemcpyAsync(st.first, first.data(), sizeof(uint32_t) * nw, hipMemcpyHostToDevice, s));
+    SRT_HIP_TRY(launch_stream_fill(nw, st.R, st.V, st.waves, pk.K, st.rows_of, pk.col_ptr, pk.cols, pk.vals, d_blk,
+                                   st.first, st.blocks, s));
+    SRT_HIP_TRY(hipStreamSynchronize(s));
+    st.bytes = sizeof(uint32_t) * (words + nw) + sizeof(int32_t) * rows.size();
+    out = st;
+    guard.p = nullptr;
+    return SRT_OK;
+}
+
 // Column / value arrays of pk.total_cols / pk.total_vals entries plus the
 // zeroed tail padding the executor's batch reads rely on.
 static int alloc_packed_arrays(Packed &pk, hipStream_t s) {
@@ -1197,6 +1316,25 @@ static bool full_pattern(const ExecutorDesc *e) {
     return e && e->M_r == 4 && e->num_patterns == 1 && e->patterns[0] == 15;
 }
 
+// The gather schedule of a streamed plan (grouped and persistent launches run
+// it), built at the first need; other plans have it from their creation.
+static int ensure_gather(const srt_plan *cp) {
+    if (!streamed(cp->cfg)) return SRT_OK;
+    srt_plan *p = const_cast<srt_plan *>(cp);
+    std::lock_guard<std::mutex> g(p->mu);
+    if (p->sch.desc) return SRT_OK;
+    srt_tile_config c = p->cfg_user;
+    c.b_staging = 2;
+    c.chunk_cols = c.nsplit = 0;
+    const int n = std::max(p->n_max, 1);
+    realise_config(c, p->pk.M_r, p->pk.K, p->pk.K_c, p->pk.total_cols, n);
+    Schedule sch;
+    std::vector<RetiredSchedule> none;
+    SRT_TRY(build_schedule(p->pk, c, p->exec, config_tiles(c, n), sch, none, c, nullptr));
+    p->sch = std::move(sch);
+    return SRT_OK;
+}
+
 // Panel ranges of the matrix-core executor for B width n: R contiguous
 // ranges balanced by packed columns (+4 per panel for its C rows), R x
 // (64-column slices) = one round of 256 CUs; the ranges of a width used
@@ -1266,6 +1404,18 @@ int srt_plan_create(int m, int k, int n, const float *Lx, const void *Lp, const 
     else srt_tile_config_default(&plan->cfg_user);
     plan->n_max = n;
     plan->cfg = plan->cfg_user;
+    if (column_ordered(exec) && (plan->cfg.b_staging == 0 || plan->cfg.b_staging == 3) && plan->cfg.matrix_cores != 1 &&
+        m > 0 && k > 0) {
+        realise_stream(plan->cfg, m, k, plan->pk.K_c, plan->pk.total_cols, std::max(n, 1));
+        rc = build_stream(plan->pk, plan->cfg, plan->stream, (hipStream_t)stream);
+        if (rc) {
+            plan->pk.release();
+            return rc;
+        }
+        plan->sch.kp.assign(plan->pk.P, 1);
+        *out = plan.release();
+        return SRT_OK;
+    }
     realise_config(plan->cfg, map.M_r, k, plan->pk.K_c, plan->pk.total_cols, std::max(n, 1));
     if (plan->cfg.matrix_cores == 1) {
         if (!full_pattern(exec))
@@ -1413,12 +1563,20 @@ int srt_plan_create_hybrid(int m, int k, int n, const float *Lx, const void *Lp,
         pk.h_skip.assign((size_t)pk.P, 0);
         for (int d = 0; d < nd; ++d)
             for (int r = dense_rows[d]; r < std::min(m, dense_rows[d] + 16); r += pk.M_r) pk.h_skip[(size_t)(r / pk.M_r)] = 1;
-        Schedule first = std::move(plan->sch);
-        plan->sch = Schedule();
-        const int rc = build_schedule(pk, plan->cfg, plan->exec, config_tiles(plan->cfg, std::max(n, 1)), plan->sch,
-                                      plan->retired, plan->cfg, s);
-        first.release();
-        SRT_TRY(rc);
+        if (streamed(plan->cfg)) {
+            StreamSched first = plan->stream;
+            plan->stream = StreamSched();
+            const int rc = build_stream(pk, plan->cfg, plan->stream, s);
+            first.release();
+            SRT_TRY(rc);
+        } else {
+            Schedule first = std::move(plan->sch);
+            plan->sch = Schedule();
+            const int rc = build_schedule(pk, plan->cfg, plan->exec, config_tiles(plan->cfg, std::max(n, 1)),
+                                          plan->sch, plan->retired, plan->cfg, s);
+            first.release();
+            SRT_TRY(rc);
+        }
     }
     plan->pk.nnz = nnz;  // the whole matrix's entries (the register-tiled part holds the others)
     *out = guard.release();
@@ -1455,6 +1613,19 @@ int srt_plan_allocate_executor(srt_plan *p, int n) {
     // schedule (schedules of other widths stay alive: graphs captured with
     // them replay unchanged).  Not concurrently with other calls on the plan.
     srt_tile_config c = p->cfg_user;
+    if (streamed(p->cfg)) {
+        realise_stream(c, p->pk.M, p->pk.K, p->pk.K_c, p->pk.total_cols, std::max(n, 1));
+        if (c.vec_width == p->stream.V && c.waves_per_block == p->stream.waves && c.chunk_cols == p->stream.R)
+            return SRT_OK;
+        if (!p->pk.cols && p->pk.total_cols)
+            return fail(SRT_ERR_INVALID, "the plan's column indices were released: its schedule cannot change");
+        StreamSched st;
+        SRT_TRY(build_stream(p->pk, c, st, nullptr));
+        p->retired_streams.push_back(p->stream);
+        p->stream = st;
+        p->cfg = c;
+        return SRT_OK;
+    }
     realise_config(c, p->pk.M_r, p->pk.K, p->pk.K_c, p->pk.total_cols, std::max(n, 1));
     const int tiles = config_tiles(c, std::max(n, 1));
     srt_tile_config sch_cfg = p->cfg;
@@ -1473,7 +1644,9 @@ int srt_plan_execute(const srt_plan *p, float *C, int64_t ldc, const float *B, i
     // With every 16-row panel dense the register-tiled part is empty and the
     // dense panels write every row of C.
     const bool all_dense = p->dense.ndense > 0 && (int64_t)p->dense.ndense * 16 >= p->pk.M;
-    if (all_dense || p->cfg.matrix_cores == 1) {
+    if (streamed(p->cfg) && !all_dense) {
+        SRT_TRY(run_stream(p->pk, p->stream, p->cfg, B, ldb, C, ldc, n, (hipStream_t)stream));
+    } else if (all_dense || p->cfg.matrix_cores == 1) {
         if (n < 0) return fail(SRT_ERR_INVALID, "n must be >= 0");
         if (n > 0 && (!B || !C)) return fail(SRT_ERR_INVALID, "null B or C");
         if (n > 0 && (ldb < n || ldc < n)) return fail(SRT_ERR_INVALID, "ldb and ldc must be >= n");
@@ -1499,6 +1672,7 @@ int srt_plan_release_columns(srt_plan *p) {
     if (!p) return fail(SRT_ERR_INVALID, "null plan");
     if (p->cfg.matrix_cores == 1)
         return fail(SRT_ERR_UNSUPPORTED, "matrix-core execution reads the column indices at every launch");
+    SRT_TRY(ensure_gather(p));  // it cannot be built later
     SRT_HIP_TRY(hipDeviceSynchronize());  // no launch that builds a schedule may still read them
     (void)hipFree(p->pk.cols);
     p->pk.cols = nullptr;
@@ -1507,7 +1681,7 @@ int srt_plan_release_columns(srt_plan *p) {
 
 int srt_plan_schedule_bytes(const srt_plan *p, size_t *bytes) {
     if (!p || !bytes) return fail(SRT_ERR_INVALID, "null argument");
-    *bytes = p->sch.bytes;
+    *bytes = p->sch.bytes + p->stream.bytes;
     return SRT_OK;
 }
 
@@ -1515,6 +1689,11 @@ int srt_plan_launch_shape(const srt_plan *p, int n, int *grid, int *block) {
     if (!p || n < 0) return fail(SRT_ERR_INVALID, "null plan or negative n");
     const int V = std::max(1, p->cfg.vec_width);
     const int64_t tiles = ((int64_t)n + 64 * V - 1) / (64 * V);
+    if (streamed(p->cfg)) {
+        if (grid) *grid = (int)std::min<int64_t>((int64_t)p->stream.n_wg * tiles, 0x7fffffff);
+        if (block) *block = 64 * p->stream.waves;
+        return SRT_OK;
+    }
     if (grid) *grid = (int)std::min<int64_t>((int64_t)p->sch.n_wblocks * tiles, 0x7fffffff);
     if (block) *block = 64 * p->sch.waves_per_block;
     return SRT_OK;
@@ -1568,6 +1747,8 @@ void srt_plan_destroy(srt_plan *p) {
     p->pk.release();
     p->sch.release();
     for (RetiredSchedule &r : p->retired) r.sch.release();
+    p->stream.release();
+    for (StreamSched &st : p->retired_streams) st.release();
     p->dense.release();
     for (auto &r : p->mfma_ranges) (void)hipFree(r.second);
     delete p;
@@ -1666,6 +1847,7 @@ int srt_group_create(const srt_plan *const *plans, int count, const float *const
     SRT_HIP_TRY(hipGetDevice(&g->device));
     for (int i = 0; i < count; ++i) {
         const srt_plan *p = plans[i];
+        SRT_TRY(ensure_gather(p));
         if (p->device != g->device) return fail(SRT_ERR_INVALID, "srt_group_create: plan belongs to another device");
         if (p->dense.ndense) return fail(SRT_ERR_UNSUPPORTED, "srt_group_create: hybrid plans execute alone");
         if (i == 0) {
@@ -1725,6 +1907,7 @@ int srt_exec_problem_fill(const srt_plan *p, const float *B, int64_t ldb, float 
     const int V = vec_width;
     if (V != 1 && V != 2 && V != 4) return fail(SRT_ERR_INVALID, "vec_width must be 1, 2 or 4");
     if (n < 0 || ldb < n || ldc < n || block_begin < 0) return fail(SRT_ERR_INVALID, "bad n / ldb / ldc / block_begin");
+    SRT_TRY(ensure_gather(p));
     if (p->sch.unroll != kPersistentUnroll)
         return fail(SRT_ERR_UNSUPPORTED, "the plan's schedule is not cut for unroll 4 (TileConfig.unroll = 4)");
     if (p->dense.ndense) return fail(SRT_ERR_UNSUPPORTED, "hybrid plans execute alone");
@@ -1765,6 +1948,7 @@ int srt_exec_persistent_execute(const srt_plan *proto, int vec_width, const srt_
     const int V = vec_width;
     if (V != 1 && V != 2 && V != 4) return fail(SRT_ERR_INVALID, "vec_width must be 1, 2 or 4");
     if (grid < 1) return fail(SRT_ERR_INVALID, "grid must be >= 1");
+    SRT_TRY(ensure_gather(proto));
     if (proto->sch.unroll != kPersistentUnroll)
         return fail(SRT_ERR_UNSUPPORTED, "the plan's schedule is not cut for unroll 4 (TileConfig.unroll = 4)");
     int dev = -1;

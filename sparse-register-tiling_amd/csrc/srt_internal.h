@@ -159,6 +159,36 @@ struct RetiredSchedule {
     Schedule sch;
 };
 
+// Streamed execution (stream_exec.hip) of a column-ordered packing (M_r = 1):
+// entry blocks per stream wave, the C rows of each, for one launch shape.
+struct StreamSched {
+    uint32_t *blocks = nullptr;   // device: per block S values, then S LDS offsets
+    uint32_t *first = nullptr;    // device: first block of each wave
+    int32_t *rows_of = nullptr;   // device: [n_wg * waves * R] C row or -1
+    int V = 0, waves = 0, R = 0, n_wg = 0;
+    size_t bytes = 0;
+    void release();
+};
+
+struct StreamLaunch {
+    const uint32_t *blocks, *first;
+    const int32_t *rows_of;
+    const float *B;
+    float *C;
+    int64_t ldb, ldc;
+    int N, K, V, R, waves, n_wg, xcd_remap;
+};
+
+int stream_tile_rows(int V, int waves);   // B rows of one LDS tile
+int stream_block_words(int V);            // words of one entry block
+hipError_t launch_stream(const StreamLaunch &a, hipStream_t s);
+hipError_t launch_stream_count(int n_waves, int R, int V, int waves, int K, const int32_t *rows_of,
+                               const int64_t *col_ptr, const int32_t *cols, int32_t *tile_blocks, uint32_t *total,
+                               hipStream_t s);
+hipError_t launch_stream_fill(int n_waves, int R, int V, int waves, int K, const int32_t *rows_of,
+                              const int64_t *col_ptr, const int32_t *cols, const float *vals,
+                              const int32_t *tile_blocks, const uint32_t *first, uint32_t *blocks, hipStream_t s);
+
 // Kernel launchers (packer.hip).
 // CSR packing in O(nnz) memory (packer.hip): cell keys, radix sort, cells,
 // segment bounds, per-segment counts and fill.  The two hipcub-backed steps

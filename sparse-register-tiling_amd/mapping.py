@@ -250,6 +250,9 @@ def identity_strategy(M_r: int) -> SOPOrig:
 
 STRATEGIES: Dict[str, Callable[[], SOPOrig]] = {
     # name -> strategy; the id each one produces is checked by the tests.
+    # M_r=1: one row per panel, so a chain is the row's nonzeros in column
+    # order; what the streamed executor runs.
+    "M1_identity": lambda: identity_strategy(1),
     "M2_identity": lambda: identity_strategy(2),
     "M4_identity": lambda: identity_strategy(4),
     "M6_identity": lambda: identity_strategy(6),
@@ -267,12 +270,12 @@ STRATEGIES: Dict[str, Callable[[], SOPOrig]] = {
     "M8_alt": lambda: SOPOrig(_M8_MERGE, [1 << i for i in range(8)], split_cost=10000),
 }
 
-STRATEGY_M_R = {"M2_identity": 2, "M4_identity": 4, "M6_identity": 6, "M8_identity": 8,
+STRATEGY_M_R = {"M1_identity": 1, "M2_identity": 2, "M4_identity": 4, "M6_identity": 6, "M8_identity": 8,
                 "M4_orig": 4, "M4_full": 4, "M8_orig": 8, "M8_alt": 8}
 
 # tools/paper/configs.py:84-87, plus the identity mappings of the other
 # panel heights (sbench/SOP/identity_mappings/{2,6,8}).
-NAMED_IDS = {2: {"identity": "4af51"}, 4: {"identity": "61fee", "orig": "da01e", "full": "7da09"},
+NAMED_IDS = {1: {"identity": "2b3d8"}, 2: {"identity": "4af51"}, 4: {"identity": "61fee", "orig": "da01e", "full": "7da09"},
              6: {"identity": "001e3"}, 8: {"orig": "400fa", "alt": "747f9", "identity": "161fb"}}
 
 

@@ -1,0 +1,129 @@
+"""Streamed execution (M_r = 1, tiles of B rows in LDS): bit-identical to the
+sequential fused multiply-add chain over each row's nonzeros in column order
+(the oracle's CSR executor) at the edges of tiles, slices, waves and quads."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _plan(srt, torch, A, n, index_dtype=np.int64, **cfg):
+    rp, ci, v = srt.workloads.to_csr(A, index_dtype)
+    return srt.MatMulSpecialized(A.shape[0], A.shape[1], n, torch.from_numpy(v), torch.from_numpy(rp),
+                                 torch.from_numpy(ci), tile_config=srt.TileConfig(b_staging=3, **cfg),
+                                 mapping_id=srt.named_mapping(1, "identity"))
+
+
+def _chain(srt, cb, A, B):
+    rp, ci, v = srt.workloads.to_csr(A)
+    return cb.csr_exec(rp, ci, v, A.shape[0], B)
+
+
+def _same(C, ref):
+    assert np.array_equal(np.isnan(C), np.isnan(ref))
+    ok = ~np.isnan(ref)
+    assert np.array_equal(C.view(np.uint32)[ok], ref.view(np.uint32)[ok])
+
+
+# tile edges: V = 4 holds 64 rows at 16 waves (32 at 8), V = 2 128, V = 1 256
+CASES = [(1, 1, 1), (17, 63, 5), (64, 64, 256), (33, 65, 257), (130, 129, 64), (70, 255, 131), (257, 300, 510),
+         (40, 513, 1023), (300, 777, 333), (16, 2048, 96)]
+
+
+@pytest.mark.parametrize("V,W,R", [(1, 16, 1), (1, 4, 8), (2, 16, 2), (2, 8, 4), (4, 16, 8), (4, 16, 1), (4, 4, 2),
+                                   (4, 8, 4), (0, 0, 0)])
+@pytest.mark.parametrize("M,K,N", CASES)
+def test_bitexact_at_the_edges(srt, oracle, M, K, N, V, W, R):
+    import torch
+    _, cb = oracle
+    rng = np.random.default_rng(M * 7 + K * 3 + N)
+    A = (rng.standard_normal((M, K)) * (rng.random((M, K)) < 0.3)).astype(np.float32)
+    A[:: max(1, M // 5)] = 0  # empty rows
+    A[M // 2] = rng.standard_normal(K)  # a full one
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    print("case", M, K, N, V, W, R, flush=True)
+    plan = _plan(srt, torch, A, N, np.int32 if N % 2 else np.int64, vec_width=V, waves_per_block=W, chunk_cols=R)
+    real = plan.get_config()
+    assert real.b_staging == 3 and (not V or (real.vec_width, real.waves_per_block, real.chunk_cols) == (V, W, R))
+    wide = torch.full((K, N + 5), 9.0, device="cuda")  # strided, unaligned rows
+    wide[:, 3:3 + N] = torch.from_numpy(B).cuda()
+    C = torch.full((M, N + 3), float("nan"), device="cuda")
+    plan(C[:, 1:], wide[:, 3:3 + N], n=N)
+    torch.cuda.synchronize()
+    got = C.cpu().numpy()
+    _same(np.ascontiguousarray(got[:, 1:1 + N]), _chain(srt, cb, A, B))
+    assert np.isnan(got[:, 0]).all() and np.isnan(got[:, 1 + N:]).all()
+
+
+def test_values_that_are_not_numbers(srt, oracle):
+    """Padding leaves infinities, NaN and signed zeros as the chain has them."""
+    import torch
+    _, cb = oracle
+    rng = np.random.default_rng(5)
+    A = (rng.standard_normal((64, 200)) * (rng.random((64, 200)) < 0.2)).astype(np.float32)
+    B = rng.uniform(-1, 1, (200, 70)).astype(np.float32)
+    A[3, 7], A[4, 9], A[5, :] = np.inf, -np.inf, 0
+    A[5, 11] = np.float32(-1e-30)
+    B[20, 3], B[21, 4], B[11] = np.inf, np.nan, np.float32(1e-30)  # row 5: -0 by underflow
+    plan = _plan(srt, torch, A, 70)
+    C = torch.empty((64, 70), device="cuda")
+    plan(C, torch.from_numpy(B).cuda())
+    _same(C.cpu().numpy(), _chain(srt, cb, A, B))
+
+
+def test_other_widths_groups_and_graphs(srt, oracle):
+    """One plan at other widths, rebuilt for one, captured, in a group, as a hybrid."""
+    import torch
+    _, cb = oracle
+    A = srt.workloads.magnitude_pruned(200, 150, 0.7, seed=3)
+    plan = _plan(srt, torch, A, 256)
+    B = srt.workloads.dense_b(150, 300, seed=4)
+    Bt = torch.from_numpy(B).cuda()
+    ref = _chain(srt, cb, A, B)
+    C = torch.empty((200, 300), device="cuda")
+    for n in (300, 1, 64, 257):
+        plan(C, Bt, n=n)
+        _same(np.ascontiguousarray(C.cpu().numpy()[:, :n]), np.ascontiguousarray(ref[:, :n]))
+    plan.allocate_executor(8)
+    plan(C, Bt)
+    _same(C.cpu().numpy(), ref)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        plan(C, Bt)
+    for _ in range(3):
+        C.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        _same(C.cpu().numpy(), ref)
+    two = _plan(srt, torch, A, 300)
+    C2 = torch.empty_like(C)
+    grp = srt.cnn.GroupedPlans([plan, two], [Bt, Bt], [C, C2])  # the gather schedules, built on demand
+    C.zero_()
+    grp()
+    torch.cuda.synchronize()
+    assert np.allclose(C.cpu().numpy(), ref, rtol=0, atol=1e-4) and torch.equal(C, C2)
+    grp.close()
+    rp, ci, v = srt.workloads.to_csr(A)
+    h = srt.MatMulSpecialized(200, 150, 300, torch.from_numpy(v), torch.from_numpy(rp), torch.from_numpy(ci),
+                              mapping_id=srt.named_mapping(1, "identity"), dense_threshold=0.35)
+    dense = h.dense_panels()["rows"]
+    assert 0 < len(dense) < 13
+    h(C, Bt)
+    rest = np.ones(200, dtype=bool)
+    for r in dense:
+        rest[r:r + 16] = False
+    got = C.cpu().numpy()
+    _same(np.ascontiguousarray(got[rest]), np.ascontiguousarray(ref[rest]))
+    assert np.all(np.abs(got - cb.dense_f64(A, B)) <= srt_bound(A, B))
+
+
+def srt_bound(A, B):
+    """FP32 summation bound of a chain: 2 L 2^-24 (|A| |B|)."""
+    L = int((A != 0).sum(axis=1).max())
+    return 2 * L * 2.0 ** -24 * (np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64)) + 1e-30
+
+
+def test_rule_takes_streams_for_much_work(srt):
+    at = srt.autotune
+    assert at.streamed_launch(4096, 1024, 838860, 2048)[2] < at.gather_seconds(4096, 1024, 838860, 2048)
+    assert at.streamed_launch(512, 512, 13107, 8)[2] > at.gather_seconds(512, 512, 13107, 8)
