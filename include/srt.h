@@ -308,7 +308,8 @@ int srt_group_create(const srt_plan *const *plans, int count, const float *const
 int srt_group_rebind(srt_group *g, const float *const *B, const int64_t *ldb, float *const *C,
                      const int64_t *ldc, const int *n, srt_stream_t stream);
 int srt_group_execute(const srt_group *g, srt_stream_t stream);
-/* Lane width (floats per lane) of the launch, workgroups, LDS bytes. */
+/* Lane width (floats per lane) of the group's narrowest problem (each runs at
+ * its own), workgroups, LDS bytes. */
 int srt_group_info(const srt_group *g, int *vec_width, int *workgroups, int *lds_bytes);
 void srt_group_destroy(srt_group *g);
 

@@ -76,7 +76,7 @@ struct Dispatch {{
     static __device__ __forceinline__ void fmas(int key, float (&acc)[MR][V],
                                                 const typename srt::VecOf<V>::type (&rows)[U],
                                                 const float (&vals)[srt::kValWindow],
-                                                const float *__restrict__ vp) {{
+                                                srt::ConstPtr<float> vp) {{
         static_assert(U == {U}, "one unroll per translation unit");
         switch (key) {{
 {cases}

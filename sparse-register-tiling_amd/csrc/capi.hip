@@ -553,7 +553,7 @@ static int log2_small(int v) { return v >= 8 ? 3 : v >= 4 ? 2 : v >= 2 ? 1 : 0; 
 static bool pow2_upto8(int v) { return v == 1 || v == 2 || v == 4 || v == 8; }
 
 static constexpr int kMaxWaves = 16;        // wave slots per workgroup (launch bound 1024)
-static constexpr size_t kMaxLdsL2 = 65536;  // reduction LDS of the global-memory B path
+static constexpr size_t kMaxLdsL2 = 131072;  // reduction LDS of the global-memory B path: 16 waves of 8 rows, V = 4
 
 static size_t reduce_lds(int waves, int M_r, int V) { return (size_t)waves * M_r * V * 64 * sizeof(float); }
 static size_t tile_lds(int K, int V) { return (size_t)K * 64 * V * sizeof(float); }
@@ -596,10 +596,23 @@ static int cu_count() {
 // `total_cols` packed columns and B width n (the choices the reference's
 // heuristic JSON made per sparsity bucket are made here from the launch
 // geometry; the autotuner overrides them with measured choices).
-static void realise_config(srt_tile_config &c, int M_r, int K, int K_tile, int64_t total_cols, int n) {
-    if (c.vec_width != 1 && c.vec_width != 2 && c.vec_width != 4)
-        c.vec_width = (n % 4 == 0 && n >= 256) ? 4 : (n % 2 == 0 && n >= 128) ? 2 : 1;
-    if (c.waves_per_block < 1 || c.waves_per_block > kMaxWaves) c.waves_per_block = 8;
+//
+// Lane width: the widest whose N tiles still give the chip a workgroup per CU
+// (a panel never spans two workgroups), since a wide lane gathers the same
+// bytes in fewer batches.  Both sides at 16 waves, 8-row "orig": 4096 x 1024
+// at 90 % x 200 runs 19.5 us at V = 4 (512 workgroups) and 31.6 at V = 1;
+// 1000 x 777 at 80 % x 200 runs 12.4 at V = 1 and 16.1 at V = 4 (125).  Two
+// floats pay only with half a round more.  Waves: 16 beat 8 at 62 of 72
+// sizes (M 256-4096, K 512-4096, N 8-1024), by a tenth at the middle one,
+// and lose at most 6 %.
+static void realise_config(srt_tile_config &c, int P, int M_r, int K, int K_tile, int64_t total_cols, int n) {
+    if (c.vec_width != 1 && c.vec_width != 2 && c.vec_width != 4) {
+        const int64_t cus = cu_count();
+        c.vec_width = n > 128 && 16 * (int64_t)P * ((n + 255) / 256) >= 15 * cus ? 4
+                      : n > 64 && 2 * (int64_t)P * ((n + 127) / 128) >= 3 * cus  ? 2
+                                                                                 : 1;
+    }
+    if (c.waves_per_block < 1 || c.waves_per_block > kMaxWaves) c.waves_per_block = 16;
     if (c.nsplit < 1 || c.nsplit > c.waves_per_block) c.nsplit = c.waves_per_block;
     // B path: global-memory rows unless the LDS tile is asked for and its
     // narrowest form (V = 1) fits (measured faster on the pruned-FFN shapes).
@@ -664,6 +677,17 @@ static void realise_stream(srt_tile_config &c, int M, int K, int K_tile, int64_t
 
 static bool aligned(const void *p, int bytes) { return ((uintptr_t)p % (uintptr_t)bytes) == 0; }
 
+// The widest lane at most V for a launch.  The gather path takes any n >= V
+// and any 4-byte aligned rows: its last lane moves back to column n - V.  A
+// staged tile is read, and a C that is added to is loaded, at the lane's own
+// columns: those need V | n, ldb, ldc and 4V-byte aligned B and C.
+static int lane_width(int V, bool own_columns, int n, int64_t ldb, int64_t ldc, const void *B, const void *C) {
+    if (own_columns)
+        while (V > 1 && (n % V || ldb % V || ldc % V || !aligned(B, 4 * V) || !aligned(C, 4 * V))) V >>= 1;
+    while (V > n) V >>= 1;
+    return V;
+}
+
 static int run_executor(const Packed &pk, const Schedule &sch, const ExecutorDesc *exec,
                         const srt_tile_config &cfg, const float *B, int64_t ldb, float *C,
                         int64_t ldc, int n, int load_c, hipStream_t s) {
@@ -674,9 +698,6 @@ static int run_executor(const Packed &pk, const Schedule &sch, const ExecutorDes
     if (!sch.desc || sch.waves_per_block < 1 || sch.waves_per_block > kMaxWaves)
         return fail(SRT_ERR_INVALID, "no launch schedule");
     int V = cfg.vec_width;
-    // Vector loads need V | n, V | ldb, V | ldc and 4V-byte aligned B and C.
-    while (V > 1 && (n % V || ldb % V || ldc % V || !aligned(B, 4 * V) || !aligned(C, 4 * V)))
-        V >>= 1;
     bool stage = cfg.b_staging == 1 && tile_lds(pk.K, 1) <= lds_limit();
     if (stage) {  // executors built at run time may hold the global-memory path only
         bool any = false;
@@ -684,6 +705,7 @@ static int run_executor(const Packed &pk, const Schedule &sch, const ExecutorDes
             for (int u = 0; u < 4; ++u) any = any || exec->launch[1][v][u] != nullptr;
         stage = any;
     }
+    V = lane_width(V, stage || load_c, n, ldb, ldc, B, C);
     while (V > 1 && !lds_fits(stage, pk.K, sch.waves_per_block, pk.M_r, V, sch.reduce)) V >>= 1;
     if (stage && !lds_fits(true, pk.K, sch.waves_per_block, pk.M_r, V, sch.reduce)) stage = false;
     if (!lds_fits(stage, pk.K, sch.waves_per_block, pk.M_r, V, sch.reduce))
@@ -1327,7 +1349,7 @@ static int ensure_gather(const srt_plan *cp) {
     c.b_staging = 2;
     c.chunk_cols = c.nsplit = 0;
     const int n = std::max(p->n_max, 1);
-    realise_config(c, p->pk.M_r, p->pk.K, p->pk.K_c, p->pk.total_cols, n);
+    realise_config(c, p->pk.P, p->pk.M_r, p->pk.K, p->pk.K_c, p->pk.total_cols, n);
     Schedule sch;
     std::vector<RetiredSchedule> none;
     SRT_TRY(build_schedule(p->pk, c, p->exec, config_tiles(c, n), sch, none, c, nullptr));
@@ -1416,7 +1438,7 @@ int srt_plan_create(int m, int k, int n, const float *Lx, const void *Lp, const 
         *out = plan.release();
         return SRT_OK;
     }
-    realise_config(plan->cfg, map.M_r, k, plan->pk.K_c, plan->pk.total_cols, std::max(n, 1));
+    realise_config(plan->cfg, plan->pk.P, map.M_r, k, plan->pk.K_c, plan->pk.total_cols, std::max(n, 1));
     if (plan->cfg.matrix_cores == 1) {
         if (!full_pattern(exec))
             rc = fail(SRT_ERR_UNSUPPORTED, "matrix_cores needs M_r = 4 and a mapping whose only kernel pattern is 15");
@@ -1626,7 +1648,7 @@ int srt_plan_allocate_executor(srt_plan *p, int n) {
         p->cfg = c;
         return SRT_OK;
     }
-    realise_config(c, p->pk.M_r, p->pk.K, p->pk.K_c, p->pk.total_cols, std::max(n, 1));
+    realise_config(c, p->pk.P, p->pk.M_r, p->pk.K, p->pk.K_c, p->pk.total_cols, std::max(n, 1));
     const int tiles = config_tiles(c, std::max(n, 1));
     srt_tile_config sch_cfg = p->cfg;
     SRT_TRY(switch_schedule(p->pk, c, tiles, p->exec, p->sch, sch_cfg, p->retired, nullptr));
@@ -1760,35 +1782,40 @@ void srt_plan_destroy(srt_plan *p) {
 struct srt_group {
     std::vector<const srt_plan *> plans;
     const ExecutorDesc *exec = nullptr;
-    int waves = 0, V = 1, total_blocks = 0, xcd_remap = 1, device = 0;
+    int waves = 0, V = 1, least = 1, total_blocks = 0, xcd_remap = 1, device = 0;
     size_t lds = 0;
     ExecProblem *d_probs = nullptr;
     std::vector<ExecProblem> h_probs;
 };
 
-// Problem table of a group for the given operands: the lane width is the
-// widest every problem allows (alignment, V | n, LDS of its reduction), each
-// problem gets n_wblocks * ceil(n / 64V) consecutive workgroups.
+// Problem table of a group for the given operands: each problem runs at its
+// own lane width (the widest of the plans' that its n fills and the LDS of its
+// reduction allows) and gets n_wblocks * ceil(n / 64 lanes) consecutive
+// workgroups; the launch is the widest problem's.
 static int group_bind(srt_group &g, const float *const *B, const int64_t *ldb, float *const *C, const int64_t *ldc,
                       const int *n, hipStream_t s) {
     if (!B || !ldb || !C || !ldc || !n) return fail(SRT_ERR_INVALID, "srt_group: null operand array");
     const int cnt = (int)g.plans.size();
-    int V = 4;
-    for (int i = 0; i < cnt; ++i) V = std::min(V, g.plans[i]->cfg.vec_width);
+    int most = 4;
+    for (int i = 0; i < cnt; ++i) most = std::min(most, g.plans[i]->cfg.vec_width);
+    std::vector<int> lanes((size_t)cnt, 1);
+    int V = 1, least = 4;
     for (int i = 0; i < cnt; ++i) {
         const srt_plan &p = *g.plans[i];
         if (n[i] < 0) return fail(SRT_ERR_INVALID, "srt_group: n must be >= 0");
+        int v = n[i] > 128 ? most : std::min(most, n[i] > 64 ? 2 : 1);
         if (n[i] > 0 && p.pk.M > 0) {
             if (!B[i] || !C[i]) return fail(SRT_ERR_INVALID, "srt_group: null B or C");
             if (ldb[i] < n[i] || ldc[i] < n[i]) return fail(SRT_ERR_INVALID, "srt_group: ldb and ldc must be >= n");
             if ((int64_t)p.pk.K * ldb[i] * (int64_t)sizeof(float) > (int64_t)0xffffffffLL)
                 return fail(SRT_ERR_UNSUPPORTED, "srt_group: B larger than 4 GiB (K * ldb * 4 bytes)");
-            while (V > 1 && (n[i] % V || ldb[i] % V || ldc[i] % V || !aligned(B[i], 4 * V) || !aligned(C[i], 4 * V)))
-                V >>= 1;
         }
-        while (V > 1 && !lds_fits(false, p.pk.K, g.waves, p.pk.M_r, V, p.sch.reduce)) V >>= 1;
-        if (!lds_fits(false, p.pk.K, g.waves, p.pk.M_r, V, p.sch.reduce))
+        while (v > 1 && !lds_fits(false, p.pk.K, g.waves, p.pk.M_r, v, p.sch.reduce)) v >>= 1;
+        if (!lds_fits(false, p.pk.K, g.waves, p.pk.M_r, v, p.sch.reduce))
             return fail(SRT_ERR_UNSUPPORTED, "srt_group: chunk reduction needs more LDS than a workgroup has");
+        lanes[i] = v;
+        V = std::max(V, v);
+        least = std::min(least, v);
     }
     std::vector<ExecProblem> t;
     int64_t total = 0;
@@ -1812,9 +1839,10 @@ static int group_bind(srt_group &g, const float *const *B, const int64_t *ldb, f
         q.reduce = p.sch.reduce;
         q.load_c = 0;
         q.block_begin = (int)total;
-        total += (int64_t)p.sch.n_wblocks * ((n[i] + 64 * V - 1) / (64 * V));
+        q.lanes = lanes[i];
+        total += (int64_t)p.sch.n_wblocks * ((n[i] + 64 * lanes[i] - 1) / (64 * lanes[i]));
         if (total > 0x7fffffffLL) return fail(SRT_ERR_UNSUPPORTED, "srt_group: more than 2^31 workgroups");
-        if (p.sch.reduce) lds = std::max(lds, reduce_lds(g.waves, p.pk.M_r, V));
+        if (p.sch.reduce) lds = std::max(lds, reduce_lds(g.waves, p.pk.M_r, lanes[i]));
         t.push_back(q);
     }
     if (t.size() > g.h_probs.size() || !g.d_probs) {
@@ -1829,6 +1857,7 @@ static int group_bind(srt_group &g, const float *const *B, const int64_t *ldb, f
     }
     g.h_probs = std::move(t);
     g.V = V;
+    g.least = least;
     g.total_blocks = (int)total;
     g.lds = lds;
     return SRT_OK;
@@ -1965,7 +1994,7 @@ int srt_exec_persistent_execute(const srt_plan *proto, int vec_width, const srt_
 
 int srt_group_info(const srt_group *g, int *vec_width, int *workgroups, int *lds_bytes) {
     if (!g) return fail(SRT_ERR_INVALID, "null group");
-    if (vec_width) *vec_width = g->V;
+    if (vec_width) *vec_width = g->least;
     if (workgroups) *workgroups = g->total_blocks;
     if (lds_bytes) *lds_bytes = (int)g->lds;
     return SRT_OK;
@@ -2223,7 +2252,7 @@ int srt_tile_execute(const srt_tile *t, int N_c, const float *B, int64_t ldb, fl
     srt_tile_config c;
     if (cfg) c = *cfg;
     else srt_tile_config_default(&c);
-    realise_config(c, t->pk.M_r, t->pk.K, t->pk.K_c ? t->pk.K_c : t->pk.K, t->pk.total_cols, std::max(N_c, 1));
+    realise_config(c, t->pk.P, t->pk.M_r, t->pk.K, t->pk.K_c ? t->pk.K_c : t->pk.K, t->pk.total_cols, std::max(N_c, 1));
     std::lock_guard<std::mutex> g(t->mu);
     const int tiles = config_tiles(c, std::max(N_c, 1));
     SRT_TRY(switch_schedule(t->pk, c, tiles, t->exec, t->sch, t->sch_cfg, t->retired, (hipStream_t)stream));

@@ -47,6 +47,17 @@ __device__ __forceinline__ typename VecOf<V>::type load_vec(const float *p) {
     return *reinterpret_cast<const typename VecOf<V>::type *>(p);
 }
 
+// V floats at a 4-byte aligned address: one wide memory instruction as well
+// (global and buffer accesses of this chip need dword alignment only).
+template <int V>
+struct VecAt4 {
+    typedef float type __attribute__((ext_vector_type(V), aligned(4)));
+};
+template <>
+struct VecAt4<1> {
+    typedef float type;
+};
+
 template <int V>
 __device__ __forceinline__ float lane_elem(const typename VecOf<V>::type &v, int j) {
     return v[j];
@@ -101,30 +112,40 @@ __device__ __forceinline__ int xcd_swizzle(int b, int nb) {
     return x * q + (x < r ? x : r) + i;
 }
 
+// Schedule and values, read through the constant address space: nothing
+// writes them while an executor runs, which the compiler cannot see where the
+// kernel's own C stores come before a read (a persistent loop, the second of
+// two bodies).  It would then load every uniform word into vector registers:
+// the serving kernel took 94 of them instead of 70 and 164 us instead of 82
+// for a batch of 24 requests.
+template <typename T>
+using ConstPtr = const __attribute__((address_space(4))) T *;
+
 // Reads N consecutive wave-uniform words as wide vector values.  Element-wise
 // loads would be sunk by LLVM into the per-column branches that use them, so
 // each column would wait for its own scalar load; a vector load used by
 // several branches stays in front of them (one s_load_dwordx{2..16}, one wait).
+template <typename T, int W>
+struct Words {
+    typedef T type __attribute__((ext_vector_type(W), aligned(4)));
+};
 template <typename T, int N>
-__device__ __forceinline__ void load_uniform(const T *__restrict__ p, T (&out)[N]) {
+__device__ __forceinline__ void load_uniform(ConstPtr<T> p, T (&out)[N]) {
     int i = 0;
 #pragma unroll
     for (; i + 8 <= N; i += 8) {
-        T __attribute__((ext_vector_type(8))) v;
-        __builtin_memcpy(&v, p + i, sizeof(v));
+        const typename Words<T, 8>::type v = *(ConstPtr<typename Words<T, 8>::type>)(p + i);
 #pragma unroll
         for (int j = 0; j < 8; ++j) out[i + j] = v[j];
     }
     if constexpr (N % 8 >= 4) {
-        T __attribute__((ext_vector_type(4))) v;
-        __builtin_memcpy(&v, p + i, sizeof(v));
+        const typename Words<T, 4>::type v = *(ConstPtr<typename Words<T, 4>::type>)(p + i);
 #pragma unroll
         for (int j = 0; j < 4; ++j) out[i + j] = v[j];
         i += 4;
     }
     if constexpr (N % 4 >= 2) {
-        T __attribute__((ext_vector_type(2))) v;
-        __builtin_memcpy(&v, p + i, sizeof(v));
+        const typename Words<T, 2>::type v = *(ConstPtr<typename Words<T, 2>::type>)(p + i);
         out[i] = v[0];
         out[i + 1] = v[1];
         i += 2;
@@ -180,7 +201,7 @@ constexpr int kValWindow = 16;
 // FMAs of one batch of NCOL columns of pattern PAT.
 template <int PAT, int MR, int V, int U, int NCOL>
 __device__ __forceinline__ void batch_fmas(float (&acc)[MR][V], const typename VecOf<V>::type (&rows)[U],
-                                           const float (&av)[kValWindow], const float *__restrict__ vp) {
+                                           const float (&av)[kValWindow], ConstPtr<float> vp) {
     constexpr int PC = __builtin_popcount(PAT);
     constexpr int UW = kValWindow / PC < NCOL ? kValWindow / PC : NCOL;  // columns in the window
 #pragma unroll
@@ -195,8 +216,11 @@ __device__ __forceinline__ void batch_fmas(float (&acc)[MR][V], const typename V
 
 // vals + i for a record's value index (< 2^31): a 32-bit byte offset, which
 // scalar loads take as their offset operand (no 64-bit address arithmetic).
-__device__ __forceinline__ const float *value_at(const float *vals, int i) {
-    return reinterpret_cast<const float *>(reinterpret_cast<const char *>(vals) + ((uint32_t)i << 2));
+__device__ __forceinline__ ConstPtr<float> value_at(ConstPtr<float> vals, int i) {
+    return (ConstPtr<float>)((ConstPtr<char>)vals + ((uint32_t)i << 2));
+}
+__device__ __forceinline__ ConstPtr<int32_t> record_at(ConstPtr<int32_t> prog, uint32_t bytes) {
+    return (ConstPtr<int32_t>)((ConstPtr<char>)prog + bytes);
 }
 
 // Pipeline registers of one iteration.
@@ -214,11 +238,11 @@ struct Stage {
 // (rows, values, and the record after it from rp).
 template <int MR, int V, int U, class D, class R>
 __device__ __forceinline__ void pipe_step(float (&acc)[MR][V], const Stage<V, U> &in, Stage<V, U> &out, int key,
-                                          int vo, const int32_t *__restrict__ prog, uint32_t roff,
-                                          const float *__restrict__ vals, const R &bb) {
+                                          int vo, ConstPtr<int32_t> prog, uint32_t roff,
+                                          ConstPtr<float> vals, const R &bb) {
 #pragma unroll
     for (int u = 0; u < U; ++u) out.rows[u] = bb.load(in.rec[2 + u]);
-    load_uniform(reinterpret_cast<const int32_t *>(reinterpret_cast<const char *>(prog) + roff), out.rec);
+    load_uniform(record_at(prog, roff), out.rec);
     load_uniform(value_at(vals, in.rec[1]), out.vals);
     D::template fmas<V, U>(key, acc, in.rows, in.vals, value_at(vals, vo));
 }
@@ -251,20 +275,22 @@ __device__ __forceinline__ void pipe_step(float (&acc)[MR][V], const Stage<V, U>
 // The work of one (logical) workgroup b of one executor launch; shared by
 // the single-problem kernel and the grouped one.
 template <int MR, int V, int U, bool STAGE, class D>
-__device__ __forceinline__ void exec_body(float *lds, const int32_t *__restrict__ prog,
-                                          const int4 *__restrict__ desc, const float *__restrict__ vals,
+__device__ __forceinline__ void exec_body(float *lds, const int32_t *__restrict__ prog_,
+                                          const int4 *__restrict__ desc, const float *__restrict__ vals_,
                                           const float *__restrict__ B,
                                           uint32_t b_bytes, uint32_t ldb, float *__restrict__ C, int64_t ldc,
                                           int M, int N, int K, int n_wblocks, int reduce, int load_c, int b) {
     typedef typename VecOf<V>::type vec;
+    const ConstPtr<int32_t> prog = (ConstPtr<int32_t>)prog_;
+    const ConstPtr<float> vals = (ConstPtr<float>)vals_;
     const int waves = blockDim.x >> 6;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int ntile = b / n_wblocks;
     const int sb = b - ntile * n_wblocks;
-    const int4 *__restrict__ dw = desc + ((int64_t)sb * waves + wave) * 4;
+    const ConstPtr<int> dw = (ConstPtr<int>)(desc + ((int64_t)sb * waves + wave) * 4);
     int dv[16];  // descriptor and (for 2 + U <= 8) the first batch record: one scalar load
-    load_uniform(reinterpret_cast<const int *>(dw), dv);
+    load_uniform(dw, dv);
     const int4 d0 = make_int4(dv[0], dv[1], dv[2], dv[3]);
     const int4 d1 = make_int4(dv[4], dv[5], dv[6], dv[7]);
     const int p = d0.x;
@@ -272,7 +298,13 @@ __device__ __forceinline__ void exec_body(float *lds, const int32_t *__restrict_
     if (!STAGE && !reduce && !live) return;  // no barrier below
     const int n = ntile * (64 * V) + lane * V;
     const bool active = n < N;
-    const int nl = active ? n : 0;  // inactive lanes read columns 0..V-1 (in bounds)
+    // The lane's first column.  Where V does not divide N the last lane moves
+    // back to N - V: it repeats columns of the lane before it, the same chain
+    // and so the same bits, and both store them (N < V: its row has V columns
+    // all the same, see srt_exec_problem_fill).  A V = 1 launch of such an N
+    // walks its records once per 64 columns instead of once per 256: 4096 x
+    // 1024 at 90 % x 333 takes 62 us at V = 1 and 34 here.  Inactive lanes read columns 0 .. V - 1 (in bounds).
+    const int nl = !active ? 0 : STAGE || n + V <= N ? n : N >= V ? N - V : 0;
     const int kp = d1.z, j = d1.w;
     const __amdgpu_buffer_rsrc_t rsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(B), (short)0, (int)b_bytes, 0x00020000);
@@ -325,7 +357,7 @@ __device__ __forceinline__ void exec_body(float *lds, const int32_t *__restrict_
             for (int r = 0; r < MR; ++r) {
                 const int row = p * MR + r;
                 if (row < M && active) {
-                    const vec c = load_vec<V>(C + (int64_t)row * ldc + nl);
+                    const vec c = *reinterpret_cast<const typename VecAt4<V>::type *>(C + (int64_t)row * ldc + nl);
 #pragma unroll
                     for (int jj = 0; jj < V; ++jj) acc[r][jj] = lane_elem<V>(c, jj);
                 }
@@ -341,7 +373,7 @@ __device__ __forceinline__ void exec_body(float *lds, const int32_t *__restrict_
 #pragma unroll
             for (int k = 0; k < 2 + U; ++k) r0[k] = dv[8 + k];
         } else {
-            load_uniform(reinterpret_cast<const int32_t *>(reinterpret_cast<const char *>(prog) + roff), r0);
+            load_uniform(record_at(prog, roff), r0);
         }
         if (r0[0] >= 0) {
             typedef typename std::conditional<STAGE, LdsRows<V>, BRows<V>>::type Rows;
@@ -356,7 +388,7 @@ __device__ __forceinline__ void exec_body(float *lds, const int32_t *__restrict_
             Stage<V, U> s0, s1;
 #pragma unroll
             for (int u = 0; u < U; ++u) s0.rows[u] = bb.load(r0[2 + u]);
-            load_uniform(reinterpret_cast<const int32_t *>(reinterpret_cast<const char *>(prog) + roff + RB), s0.rec);
+            load_uniform(record_at(prog, roff + RB), s0.rec);
             load_uniform(value_at(vals, r0[1]), s0.vals);
             int key = r0[0], vo = r0[1];
             roff += 2 * RB;
@@ -409,7 +441,8 @@ __device__ __forceinline__ void exec_body(float *lds, const int32_t *__restrict_
 #pragma unroll
                     for (int jj = 0; jj < V; ++jj) c[jj] = acc[r][jj];
                 }
-                __builtin_nontemporal_store(c, reinterpret_cast<vec *>(C + (int64_t)row * ldc + n));
+                __builtin_nontemporal_store(typename VecAt4<V>::type(c),
+                                            reinterpret_cast<typename VecAt4<V>::type *>(C + (int64_t)row * ldc + nl));
             }
         }
     }
@@ -439,6 +472,14 @@ __global__ void __launch_bounds__(1024)
 typedef const __attribute__((address_space(4))) ExecProblem *ConstProblems;
 
 template <int MR, int V, int U, bool STAGE, class D>
+__device__ __forceinline__ void grouped_body(float *lds, ConstProblems probs, int q, int b) {
+    exec_body<MR, V, U, STAGE, D>(lds, probs[q].prog, reinterpret_cast<const int4 *>(probs[q].desc), probs[q].vals,
+                                  probs[q].B, probs[q].b_bytes, probs[q].ldb, probs[q].C, probs[q].ldc, probs[q].M,
+                                  probs[q].N, probs[q].K, probs[q].n_wblocks, probs[q].reduce, probs[q].load_c,
+                                  b - probs[q].block_begin);
+}
+
+template <int MR, int V, int U, bool STAGE, class D>
 __global__ void __launch_bounds__(1024)
     exec_grouped_kernel(ConstProblems probs, int nprob, int xcd_remap) {
     extern __shared__ float lds[];
@@ -449,11 +490,16 @@ __global__ void __launch_bounds__(1024)
         const int mid = (lo + hi + 1) >> 1;
         if (probs[mid].block_begin <= b) lo = mid; else hi = mid - 1;
     }
-    exec_body<MR, V, U, STAGE, D>(lds, probs[lo].prog, reinterpret_cast<const int4 *>(probs[lo].desc),
-                                  probs[lo].vals, probs[lo].B, probs[lo].b_bytes, probs[lo].ldb, probs[lo].C,
-                                  probs[lo].ldc, probs[lo].M,
-                                  probs[lo].N, probs[lo].K, probs[lo].n_wblocks, probs[lo].reduce,
-                                  probs[lo].load_c, b - probs[lo].block_begin);
+    // Each problem runs at its own lane width (at most V): an image of 49
+    // pixels keeps 49 of 64 lanes busy at one float per lane, 13 at four, and
+    // does not hold the wide problems to its width.  16 layers of a network,
+    // one of them of 49 columns: 97.5 us at the narrowest's width, 58.7 so.
+    const int lanes = probs[lo].lanes;
+    if constexpr (V >= 4)
+        if (lanes == 4) return grouped_body<MR, 4, U, STAGE, D>(lds, probs, lo, b);
+    if constexpr (V >= 2)
+        if (lanes == 2) return grouped_body<MR, 2, U, STAGE, D>(lds, probs, lo, b);
+    grouped_body<MR, 1, U, STAGE, D>(lds, probs, lo, b);
 }
 
 // Grouped and persistent: the problem count and the logical workgroup total

@@ -64,7 +64,7 @@ struct ExecProblem {
     uint32_t b_bytes, ldb;
     int M, N, K, n_wblocks, reduce, load_c;
     int block_begin;  // first logical workgroup of this problem
-    int pad;
+    int lanes;        // grouped launches: floats per lane of this problem (at most the launch's)
 };
 typedef hipError_t (*ExecGroupedFn)(const ExecProblem *d_probs, int nprob, int total_blocks, int waves,
                                     size_t lds, int xcd_remap, hipStream_t s);

@@ -1,0 +1,57 @@
+"""The gather executor at every width and alignment: the last lane moves back
+where the lane width does not divide N.  Bits of the oracle's chain, nothing
+written outside C's columns, B and C rows at any 4-byte address."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import _oracle_table, _plan
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M_r,name", [(4, "identity"), (8, "orig")])
+@pytest.mark.parametrize("V", [2, 4])
+@pytest.mark.parametrize("N", [1, 2, 3, 5, 127, 129, 255, 257, 259, 333])
+def test_any_width_bitexact(srt, oracle, M_r, name, V, N):
+    import torch
+    so, cb = oracle
+    A = srt.workloads.magnitude_pruned(70, 150, 0.8, seed=N)
+    B = srt.workloads.dense_b(150, N, seed=N + 1)
+    print("case", M_r, name, V, N, flush=True)
+    plan = _plan(srt, torch, A, N, M_r, name, vec_width=V, waves_per_block=8, nsplit=4, chunk_cols=16)
+    wide = torch.full((150, N + 6), float("nan"), device="cuda")
+    wide[:, 1:1 + N] = torch.from_numpy(B).cuda()
+    C = torch.full((70, N + 3), 7.0, device="cuda")
+    plan(C[:, 1:], wide[:, 1:1 + N], n=N)
+    torch.cuda.synchronize()
+    got = C.cpu().numpy()
+    ref = cb.exec_packed(cb.pack_dense(A, M_r, _oracle_table(so, M_r, name)), B, nsplit=plan.split_counts())
+    assert np.array_equal(np.ascontiguousarray(got[:, 1:1 + N]).view(np.uint32), ref.view(np.uint32))
+    assert (got[:, 0] == 7.0).all() and (got[:, 1 + N:] == 7.0).all()
+
+
+def test_group_of_widths(srt, oracle):
+    """One launch over problems of 1, 2 and 4 floats per lane, odd widths among them."""
+    import torch
+    so, cb = oracle
+    mapping = srt.resolve_mapping(srt.named_mapping(4, "orig"))
+    cfg = srt.TileConfig(vec_width=4, unroll=4, waves_per_block=8, nsplit=8)
+    shapes = [(64, 100, 49), (40, 60, 1), (96, 80, 100), (33, 128, 131), (64, 64, 512), (20, 40, 257)]
+    plans, Bs, Cs, refs = [], [], [], []
+    for i, (M, K, N) in enumerate(shapes):
+        A = srt.workloads.magnitude_pruned(M, K, 0.8, seed=i)
+        rp, ci, v = srt.workloads.to_csr(A)
+        p = srt.MatMulSpecialized(M, K, N, torch.from_numpy(v), torch.from_numpy(rp), torch.from_numpy(ci),
+                                  tile_config=cfg, mapping_id=mapping)
+        B = srt.workloads.dense_b(K, N, seed=i + 50)
+        plans.append(p)
+        Bs.append(torch.from_numpy(B).cuda())
+        Cs.append(torch.full((M, N), float("nan"), device="cuda"))
+        refs.append(cb.exec_packed(cb.pack_dense(A, 4, _oracle_table(so, 4, "orig")), B, nsplit=p.split_counts()))
+    g = srt.cnn.GroupedPlans(plans, Bs, Cs)
+    g()
+    torch.cuda.synchronize()
+    assert g.info()["vec_width"] == 1
+    for C, ref in zip(Cs, refs):
+        assert np.array_equal(C.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+    g.close()
