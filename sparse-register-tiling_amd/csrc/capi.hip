@@ -2303,8 +2303,9 @@ int srt_csr_spmm(int m, int k, int n, int64_t nnz, const void *rowptr, const voi
     if (ldb < n || ldc < n) return fail(SRT_ERR_INVALID, "ldb and ldc must be >= n");
     if (n_tile != 16 && n_tile != 32 && n_tile != 64 && n_tile != 128 && n_tile != 256)
         return fail(SRT_ERR_INVALID, "n_tile must be one of 16, 32, 64, 128, 256");
-    int V = n_tile <= 64 ? 1 : n_tile / 64;
-    while (V > 1 && (n % V || ldb % V || ldc % V || !aligned(B, 4 * V) || !aligned(C, 4 * V))) V >>= 1;
+    // n_tile is the reference's tile width; the same bits come out of every
+    // lane width, and the widest the columns fill reads B best.
+    const int V = n > 128 ? 4 : n > 64 ? 2 : 1;
     SRT_HIP_TRY(launch_csr(m, k, n, nnz, rowptr, colind, index_bytes, vals, B, ldb, C, ldc, V,
                            (hipStream_t)stream));
     return SRT_OK;

@@ -1,10 +1,18 @@
 // HIP CSR SpMM baseline: the reference's AVX-512 row-times-panel kernel
 // (sbench/SOP/_C/pytorch_csr_wrapper.cpp:70-102, dispatch :140-191) laid out
 // for 64-wide wavefronts.  One wavefront owns one row of A and a 64*V-column
-// slice of B/C; the row's column indices and values are wave-uniform (scalar
-// loads), each lane reads V consecutive B columns per stored entry and keeps
-// V fp32 accumulators.  Per output element the accumulation is one fused
+// slice of B/C; each lane reads V consecutive B columns per stored entry and
+// keeps V fp32 accumulators.  Per output element the accumulation is one fused
 // multiply-add per stored entry in storage order, like the reference.
+//
+// The row's indices and values come 64 at a time, one per lane, in one
+// coalesced load each (the next 64 while these run), and reach the wave as
+// scalars by readlane; 16 B rows are on their way while 16 are
+// multiplied.  Loads through the scalar unit, four entries at a time, left the
+// wave waiting twice (indices, then rows) for every four entries.  A row is one
+// chain, so the longest row's latency is the floor where the rows are few:
+// 2048 x 512 at 90 % x 256 takes 12.4 us (46.8 with the scalar loads at one
+// float per lane), 1024 x 4096 at 70 % x 512 132 (672).
 #include <hip/hip_runtime.h>
 
 #include "exec_kernel.h"
@@ -14,13 +22,18 @@ namespace srt {
 
 namespace {
 
-template <typename I, int V, int U>
+// B rows multiplied while as many are on their way (8: 17.9 us instead of 14.2
+// for 2048 x 512 at 90 % x 256 in a graph).
+constexpr int kBatch = 16;
+
+// BIG: B is larger than the 4 GiB a buffer descriptor and a 32-bit offset reach.
+template <typename I, int V, bool BIG>
 __global__ void __launch_bounds__(256)
     csr_kernel(int m, int k, int n, I nnz, const I *__restrict__ rowptr,
                const I *__restrict__ colind, const float *__restrict__ vals,
                const float *__restrict__ B, int64_t ldb, float *__restrict__ C, int64_t ldc,
                int row_groups) {
-    typedef typename VecOf<V>::type vec;
+    typedef typename VecAt4<V>::type vec;
     const int waves = blockDim.x >> 6;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
@@ -29,9 +42,18 @@ __global__ void __launch_bounds__(256)
     const int rg = b - ntile * row_groups;
     const int row = rg * waves + wave;
     if (row >= m) return;
+    // The lane's columns; the last lane moves back where V does not divide n
+    // (n >= V): it repeats columns of the lane before it, bit for bit.
     const int col = ntile * (64 * V) + lane * V;
     const bool active = col < n;
-    const float *__restrict__ Bp = B + (active ? col : 0);
+    const int cl = !active ? 0 : col + V <= n ? col : n - V;
+    BRows<V> rows;
+    if constexpr (!BIG) {
+        rows.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(B), (short)0,
+                                                      (int)(uint32_t)(((int64_t)(k - 1) * ldb + n) * 4), 0x00020000);
+        rows.voff = (uint32_t)cl * 4u;
+        rows.row_bytes = 1;  // offsets arrive in bytes
+    }
     float acc[V];
 #pragma unroll
     for (int j = 0; j < V; ++j) acc[j] = 0.0f;
@@ -41,38 +63,85 @@ __global__ void __launch_bounds__(256)
     I end = rowptr[row + 1];
     q = q < 0 ? 0 : (q > nnz ? nnz : q);
     end = end > nnz ? nnz : (end < q ? q : end);
-    for (; q + U <= end; q += U) {
-        vec bv[U];
-        float a[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const I c = colind[q + u];
-            const bool ok = c >= 0 && c < (I)k;
-            bv[u] = load_vec<V>(Bp + (int64_t)(ok ? c : 0) * ldb);
-            a[u] = ok ? vals[q + u] : 0.0f;
+    // Lane l holds entry l of 64: B row offset (bytes, or rows when BIG) and
+    // value; a lane without one holds row 0 and is not multiplied.
+    I c = -1;
+    float a = 0.0f;
+    auto fetch = [&](I at) {
+        c = -1;
+        if (at + lane < end) {
+            c = colind[at + lane];
+            a = vals[at + lane];
         }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int j = 0; j < V; ++j) acc[j] = __builtin_fmaf(a[u], lane_elem<V>(bv[u], j), acc[j]);
-    }
-    for (; q < end; ++q) {
-        const I c = colind[q];
+    };
+    int off = 0, val = 0;
+    auto take = [&]() {
         const bool ok = c >= 0 && c < (I)k;
-        const vec bv = load_vec<V>(Bp + (int64_t)(ok ? c : 0) * ldb);
-        const float a = ok ? vals[q] : 0.0f;
+        off = !ok ? 0 : BIG ? (int)c : (int)((uint32_t)c * ((uint32_t)ldb * 4u));
+        val = __builtin_bit_cast(int, ok ? a : 0.0f);
+    };
+    vec r0[kBatch], r1[kBatch];
+    auto load = [&](vec (&r)[kBatch], int j) {
 #pragma unroll
-        for (int j = 0; j < V; ++j) acc[j] = __builtin_fmaf(a, lane_elem<V>(bv, j), acc[j]);
+        for (int u = 0; u < kBatch; ++u) {
+            if constexpr (BIG)
+                r[u] = *reinterpret_cast<const vec *>(B + (int64_t)__builtin_amdgcn_readlane(off, j + u) * ldb + cl);
+            else
+                r[u] = rows.load(__builtin_amdgcn_readlane(off, j + u));
+        }
+    };
+    auto add = [&](const vec (&r)[kBatch], int from, int j, int count) {
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u)
+            if (u < count) {
+                const float v = __builtin_bit_cast(float, __builtin_amdgcn_readlane(from, j + u));
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    if constexpr (V == 1) acc[i] = __builtin_fmaf(v, r[u], acc[i]);
+                    else acc[i] = __builtin_fmaf(v, r[u][i], acc[i]);
+                }
+            }
+    };
+    fetch(q);
+    if (q < end) {
+        take();
+        load(r0, 0);
     }
+    for (; q + 64 < end; q += 64) {
+        fetch(q + 64);
+        load(r1, 16);
+        add(r0, val, 0, kBatch);
+        load(r0, 32);
+        add(r1, val, 16, kBatch);
+        load(r1, 48);
+        add(r0, val, 32, kBatch);
+        const int last = val;
+        take();
+        load(r0, 0);
+        add(r1, last, 48, kBatch);
+    }
+    // The last 1 to 64 entries.
+    const int left = (int)(end - q);
+    if (left > 16) load(r1, 16);
+    add(r0, val, 0, left);
+    if (left > 16) {
+        if (left > 32) load(r0, 32);
+        add(r1, val, 16, left - 16);
+    }
+    if (left > 32) {
+        if (left > 48) load(r1, 48);
+        add(r0, val, 32, left - 32);
+    }
+    if (left > 48) add(r1, val, 48, left - 48);
     if (active) {
-        vec c;
+        vec o;
         if constexpr (V == 1) {
-            c = acc[0];
+            o = acc[0];
         } else {
 #pragma unroll
-            for (int j = 0; j < V; ++j) c[j] = acc[j];
+            for (int j = 0; j < V; ++j) o[j] = acc[j];
         }
-        __builtin_nontemporal_store(c, reinterpret_cast<vec *>(C + (int64_t)row * ldc + col));
+        __builtin_nontemporal_store(o, reinterpret_cast<vec *>(C + (int64_t)row * ldc + cl));
     }
 }
 
@@ -86,8 +155,12 @@ hipError_t launch_csr_t(int m, int k, int n, int64_t nnz, const I *rowptr, const
     const long long nblocks = (long long)row_groups * n_tiles;
     if (nblocks == 0) return hipSuccess;
     if (nblocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL((csr_kernel<I, V, 4>), dim3((unsigned)nblocks), dim3(64 * waves), 0, s, m,
-                       k, n, (I)nnz, rowptr, colind, vals, B, ldb, C, ldc, row_groups);
+    if ((int64_t)k * ldb * (int64_t)sizeof(float) > (int64_t)0xffffffffLL || k < 1)
+        hipLaunchKernelGGL((csr_kernel<I, V, true>), dim3((unsigned)nblocks), dim3(64 * waves), 0, s, m, k, n, (I)nnz,
+                           rowptr, colind, vals, B, ldb, C, ldc, row_groups);
+    else
+        hipLaunchKernelGGL((csr_kernel<I, V, false>), dim3((unsigned)nblocks), dim3(64 * waves), 0, s, m, k, n, (I)nnz,
+                           rowptr, colind, vals, B, ldb, C, ldc, row_groups);
     return hipGetLastError();
 }
 

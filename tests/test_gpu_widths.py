@@ -55,3 +55,30 @@ def test_group_of_widths(srt, oracle):
     for C, ref in zip(Cs, refs):
         assert np.array_equal(C.cpu().numpy().view(np.uint32), ref.view(np.uint32))
     g.close()
+
+
+@pytest.mark.parametrize("index_dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("N", [1, 3, 63, 65, 127, 130, 255, 257, 513])
+def test_csr_rows_at_batch_edges(srt, oracle, index_dtype, N):
+    """CSR rows of every length around the kernel's batches of 16 and 64, columns in no order."""
+    import torch
+    _, cb = oracle
+    rng = np.random.default_rng(N)
+    lengths = [0, 1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 79, 80, 81, 127, 128, 129, 192, 193, 200]
+    K = 200
+    cols = [rng.permutation(K)[:l] for l in lengths]
+    rp = np.concatenate([[0], np.cumsum(lengths)]).astype(index_dtype)
+    ci = np.concatenate(cols).astype(index_dtype)
+    v = rng.standard_normal(len(ci)).astype(np.float32)
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    A = torch.sparse_csr_tensor(torch.from_numpy(rp), torch.from_numpy(ci), torch.from_numpy(v),
+                                size=(len(lengths), K)).cuda()
+    wide = torch.full((K, N + 5), float("nan"), device="cuda")
+    wide[:, 3:3 + N] = torch.from_numpy(B).cuda()
+    C = torch.full((len(lengths), N + 3), 7.0, device="cuda")
+    srt.csr.spmm(A, wide[:, 3:3 + N], C[:, 1:1 + N])
+    torch.cuda.synchronize()
+    got = C.cpu().numpy()
+    ref = cb.csr_exec(rp.astype(np.int64), ci.astype(np.int64), v, len(lengths), B)
+    assert np.array_equal(np.ascontiguousarray(got[:, 1:1 + N]).view(np.uint32), ref.view(np.uint32))
+    assert (got[:, 0] == 7.0).all() and (got[:, 1 + N:] == 7.0).all()
