@@ -48,31 +48,13 @@ __device__ __forceinline__ uint16_t to_bf16(float f) {
 }
 
 // float -> FP8 e4m3 (OCP "fn": bias 7, no infinities, max 448), round to
-// nearest even, saturating at +-448; NaN -> 0x7f.
+// nearest even, saturating at +-448; NaN -> 0x7f.  The conversion instruction
+// after a clamp; equal to the bit arithmetic of that definition for every one
+// of the 2^32 floats.
 __device__ __forceinline__ uint8_t to_e4m3(float f) {
-    const uint32_t u = __builtin_bit_cast(uint32_t, f);
-    const uint8_t sign = (uint8_t)((u >> 24) & 0x80u);
-    const uint32_t a = u & 0x7fffffffu;
-    if (a > 0x7f800000u) return 0x7f;
-    if (a >= 0x43e00000u) return sign | 0x7e;  // >= 448
-    const int e = (int)(a >> 23) - 127;
-    if (e < -6) {
-        // subnormal target: multiples of 2^-9; a * 512 is exact, rint is RNE
-        const float q = __builtin_rintf(__builtin_bit_cast(float, a) * 512.0f);
-        return sign | (uint8_t)q;  // q in [0, 8]; 8 is the smallest normal
-    }
-    uint32_t m = a & 0x7fffffu;
-    uint32_t r = m >> 20;
-    const uint32_t rem = m & 0xfffffu;
-    uint32_t ex = (uint32_t)(e + 7);
-    if (rem > 0x80000u || (rem == 0x80000u && (r & 1u))) {
-        if (++r == 8u) {
-            r = 0;
-            ++ex;
-        }
-    }
-    if (ex > 15u || (ex == 15u && r == 7u)) return sign | 0x7e;  // rounded past 448
-    return sign | (uint8_t)((ex << 3) | r);
+    const float c = __builtin_amdgcn_fmed3f(f, -448.0f, 448.0f);
+    const int w = __builtin_amdgcn_cvt_pk_fp8_f32(c, c, 0, false);
+    return f != f ? 0x7f : (uint8_t)(w & 0xff);
 }
 
 // ------------------------------------------------------------ packing
@@ -170,41 +152,102 @@ __global__ void blk_fill_kernel(int m, int k, int KB, const I *__restrict__ Lp,
 }
 
 // ------------------------------------------------------------ B operand prep
-// One block of 256 threads per 256 columns: FP8 column scales in FP64.
-__global__ void col_scale_kernel(int64_t rows, int cols, const float *__restrict__ src, int64_t ld,
-                                 float *__restrict__ scale) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= cols) return;
-    double mx = 0.0;
-    for (int64_t r = 0; r < rows; ++r) mx = fmax(mx, fabs((double)src[r * ld + c]));
-    scale[c] = mx > 0.0 ? (float)(mx / 448.0) : 1.0f;
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Columns c .. c + 4 of one row of B, zero past column `cols` (4-byte aligned
+// addresses do for a 16-byte load).
+__device__ __forceinline__ f32x4u row_quad(const float *__restrict__ row, int c, int cols) {
+    if (c + 4 <= cols) return *reinterpret_cast<const f32x4u *>(row + c);
+    f32x4u v = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (c + j < cols) v[j] = row[c + j];
+    return v;
+}
+
+// FP8 column scales max|B_j| / 448, the division in FP64 (a maximum of floats
+// is exact in FP32).  A block of 1024 threads takes 16 columns: four lanes of
+// four columns per row, 256 rows at a time, eight rows of a thread in flight.
+// Bound by the latency of its few rounds: 4096 x 512 takes 7 us; one thread
+// per column walking all rows took 1028.
+__global__ void __launch_bounds__(1024)
+    col_scale_kernel(int64_t rows, int cols, const float *__restrict__ src, int64_t ld, float *__restrict__ scale) {
+    constexpr int kRows = 8;
+    __shared__ float part[16][16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c = blockIdx.x * 16 + (threadIdx.x & 3) * 4;
+    float mx[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (c < cols)
+        for (int64_t r0 = threadIdx.x >> 2; r0 < rows; r0 += 256 * kRows) {
+            f32x4u v[kRows];
+#pragma unroll
+            for (int u = 0; u < kRows; ++u) {  // past the end: the last row again
+                const int64_t r = r0 + 256 * u < rows ? r0 + 256 * u : rows - 1;
+                v[u] = row_quad(src + r * ld, c, cols);
+            }
+#pragma unroll
+            for (int u = 0; u < kRows; ++u)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) mx[j] = fmaxf(mx[j], fabsf(v[u][j]));
+        }
+#pragma unroll
+    for (int off = 4; off < 64; off <<= 1)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) mx[j] = fmaxf(mx[j], __shfl_xor(mx[j], off));
+    if (lane < 4)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) part[wave][lane * 4 + j] = mx[j];
+    __syncthreads();
+    if (threadIdx.x < 16 && blockIdx.x * 16 + (int)threadIdx.x < cols) {
+        float m = 0.0f;
+        for (int w = 0; w < 16; ++w) m = fmaxf(m, part[w][threadIdx.x]);
+        scale[blockIdx.x * 16 + threadIdx.x] = m > 0.0f ? (float)((double)m / 448.0) : 1.0f;
+    }
 }
 
 // fp32 B (K x N, row-major) -> Bt (N x ldk, k contiguous) in BF16 or e4m3,
 // k in [K, ldk) zero: the MFMA B operand wants eight consecutive k of one
-// column per lane.  32 x 32 tiles go through LDS so that both the reads of B
-// and the writes of Bt are coalesced.
+// column per lane.  A tile of 32 columns and one 128-byte line of k per output
+// row goes through LDS: 16-byte reads of B, 16-byte writes of Bt (wide: Bt's
+// rows are 16-byte aligned).  An e4m3 value is B / scale rounded once: the
+// FP32 quotient equals the FP64 one rounded to FP32.
 template <bool FP8>
-__global__ void b_transpose_kernel(int K, int N, const float *__restrict__ src, int64_t ld_src,
-                                   const float *__restrict__ cscale, typename std::conditional<FP8, uint8_t, uint16_t>::type *__restrict__ dst,
-                                   int64_t ldk) {
-    __shared__ float t[32][33];
-    const int k0 = blockIdx.x * 32, n0 = blockIdx.y * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    for (int i = ty; i < 32; i += 8) {
-        const int k = k0 + i, n = n0 + tx;
-        t[i][tx] = (k < K && n < N) ? src[(int64_t)k * ld_src + n] : 0.0f;
+__global__ void __launch_bounds__(256)
+    b_transpose_kernel(int K, int N, const float *__restrict__ src, int64_t ld_src,
+                       const float *__restrict__ cscale, typename std::conditional<FP8, uint8_t, uint16_t>::type *__restrict__ dst,
+                       int64_t ldk, int wide) {
+    typedef typename std::conditional<FP8, uint8_t, uint16_t>::type T;
+    constexpr int TK = FP8 ? 128 : 64;   // k of a tile
+    constexpr int PER = FP8 ? 16 : 8;    // elements of 16 bytes
+    __shared__ float t[TK][33];
+    const int k0 = blockIdx.x * TK, n0 = blockIdx.y * 32;
+    f32x4u v[TK / 32];
+#pragma unroll
+    for (int i = 0; i < TK / 32; ++i) {
+        const int k = k0 + i * 32 + (threadIdx.x >> 3), n = n0 + (threadIdx.x & 7) * 4;
+        v[i] = f32x4u{0.0f, 0.0f, 0.0f, 0.0f};
+        if (k < K && n < N) v[i] = row_quad(src + (int64_t)k * ld_src, n, N);
     }
+#pragma unroll
+    for (int i = 0; i < TK / 32; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) t[i * 32 + (threadIdx.x >> 3)][(threadIdx.x & 7) * 4 + j] = v[i][j];
     __syncthreads();
-    for (int i = ty; i < 32; i += 8) {
-        const int n = n0 + i, k = k0 + tx;
-        if (n < N && k < ldk) {
-            const float v = t[tx][i];
-            if constexpr (FP8)
-                dst[(int64_t)n * ldk + k] = to_e4m3((float)((double)v / (double)cscale[n]));
-            else
-                dst[(int64_t)n * ldk + k] = to_bf16(v);
-        }
+    const int n = n0 + (threadIdx.x >> 3), kc = (threadIdx.x & 7) * PER;
+    if (n >= N || k0 + kc >= ldk) return;
+    const float s = FP8 ? cscale[n] : 1.0f;
+    T __attribute__((aligned(16))) out[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const float x = t[kc + j][threadIdx.x >> 3];
+        if constexpr (FP8) out[j] = to_e4m3(x / s);
+        else out[j] = to_bf16(x);
+    }
+    T *to = dst + (int64_t)n * ldk + k0 + kc;
+    if (wide) {
+        *reinterpret_cast<uint4 *>(to) = *reinterpret_cast<const uint4 *>(out);
+    } else {
+        for (int j = 0; j < PER && k0 + kc + j < ldk; ++j) to[j] = out[j];
     }
 }
 
@@ -560,15 +603,17 @@ hipError_t launch_mfma_fill(int m, int k, int KB, const void *Lp, const void *Li
 hipError_t launch_b_convert(int64_t rows, int cols, const float *src, int64_t ld_src, bool fp8,
                             float *cscale, void *dst, int64_t ldk, hipStream_t s) {
     if (rows <= 0 || cols <= 0) return hipSuccess;
-    const dim3 grid((unsigned)((ldk + 31) / 32), (unsigned)((cols + 31) / 32));
+    const int tk = fp8 ? 128 : 64, esz = fp8 ? 1 : 2;
+    const dim3 grid((unsigned)((ldk + tk - 1) / tk), (unsigned)((cols + 31) / 32));
+    const int wide = (uintptr_t)dst % 16 == 0 && ldk * esz % 16 == 0;
     if (fp8) {
-        hipLaunchKernelGGL(col_scale_kernel, dim3((cols + 255) / 256), dim3(256), 0, s, rows, cols, src, ld_src,
+        hipLaunchKernelGGL(col_scale_kernel, dim3((cols + 15) / 16), dim3(1024), 0, s, rows, cols, src, ld_src,
                            cscale);
         hipLaunchKernelGGL(b_transpose_kernel<true>, grid, dim3(256), 0, s, (int)rows, cols, src, ld_src, cscale,
-                           (uint8_t *)dst, ldk);
+                           (uint8_t *)dst, ldk, wide);
     } else {
         hipLaunchKernelGGL(b_transpose_kernel<false>, grid, dim3(256), 0, s, (int)rows, cols, src, ld_src,
-                           (const float *)nullptr, (uint16_t *)dst, ldk);
+                           (const float *)nullptr, (uint16_t *)dst, ldk, wide);
     }
     return hipGetLastError();
 }

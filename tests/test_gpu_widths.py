@@ -82,3 +82,31 @@ def test_csr_rows_at_batch_edges(srt, oracle, index_dtype, N):
     ref = cb.csr_exec(rp.astype(np.int64), ci.astype(np.int64), v, len(lengths), B)
     assert np.array_equal(np.ascontiguousarray(got[:, 1:1 + N]).view(np.uint32), ref.view(np.uint32))
     assert (got[:, 0] == 7.0).all() and (got[:, 1 + N:] == 7.0).all()
+
+
+@pytest.mark.parametrize("K", [1, 31, 64, 65, 127, 129, 300, 2100])
+@pytest.mark.parametrize("N", [1, 3, 16, 31, 33, 66])
+def test_operand_preparation(srt, K, N):
+    """prepare_b at the edges of its tiles, from rows at any 4-byte address:
+    transposed BF16 and e4m3 operands and column scales, bit for bit."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(K * 100 + N)
+    wide = torch.full((K, N + 5), float("nan"), device="cuda")
+    B = wide[:, 3:3 + N]
+    B.copy_(torch.randn((K, N), generator=g, device="cuda") * torch.exp(4 * torch.randn((1, N), generator=g, device="cuda")))
+    B[:, N // 2] = 0
+    ldk = -(-K // 32) * 32
+    A = torch.zeros((16, K))
+    A[0, 0] = 1
+    plans = {d: srt.precision.PanelPlan.from_dense(A, d) for d in ("bf16", "fp8")}
+    Bt, _ = plans["bf16"].prepare_b(B)
+    ref = torch.zeros((N, ldk), dtype=torch.bfloat16, device="cuda")
+    ref[:, :K] = B.t().to(torch.bfloat16)
+    assert torch.equal(Bt.view(torch.int16), ref.view(torch.int16))
+    Bq, t = plans["fp8"].prepare_b(B)
+    top = B.abs().amax(dim=0).double()
+    scale = torch.where(top > 0, (top / 448.0).float(), torch.ones_like(t))
+    assert torch.equal(t, scale)
+    q = torch.zeros((N, ldk), dtype=torch.uint8, device="cuda")
+    q[:, :K] = (B.double() / scale.double()).float().t().contiguous().to(torch.float8_e4m3fn).view(torch.uint8)
+    assert torch.equal(Bq, q)
