@@ -13,7 +13,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import _lib
-from .native import ptr, require_cuda_f32, stream_handle
+from .native import current_raw_stream, require_cuda_f32
 from .sop import MEASURED_ITERATIONS, _time_runs
 
 
@@ -22,11 +22,14 @@ def _parts(csr: torch.Tensor):
         raise ValueError("expected a torch.sparse_csr tensor")
     if csr.dim() != 2:
         raise ValueError("expected a 2-D CSR matrix")
-    rp = csr.crow_indices().cuda().contiguous()
-    ci = csr.col_indices().cuda().contiguous()
-    if ci.dtype != rp.dtype:
-        ci = ci.to(rp.dtype)
-    vals = csr.values().to(device="cuda", dtype=torch.float32).contiguous()
+    rp, ci, vals = csr.crow_indices(), csr.col_indices(), csr.values()
+    if not (csr.is_cuda and vals.dtype is torch.float32 and ci.dtype is rp.dtype and rp.is_contiguous()
+            and ci.is_contiguous() and vals.is_contiguous()):
+        rp = rp.cuda().contiguous()
+        ci = ci.cuda().contiguous()
+        if ci.dtype != rp.dtype:
+            ci = ci.to(rp.dtype)
+        vals = vals.to(device="cuda", dtype=torch.float32).contiguous()
     return rp, ci, vals
 
 
@@ -42,8 +45,10 @@ def spmm(csr: torch.Tensor, B: torch.Tensor, C: Optional[torch.Tensor] = None, n
         C = torch.empty((m, n), dtype=torch.float32, device=B.device)
     require_cuda_f32(C, "C")
     rp, ci, vals = _parts_cache or _parts(csr)
-    _lib.call("srt_csr_spmm", m, k, n, ci.numel(), ptr(rp), ptr(ci), rp.element_size(), ptr(vals),
-              ptr(B), B.stride(0), ptr(C), C.stride(0), int(n_tile), stream_handle(stream))
+    s = current_raw_stream(torch.cuda.current_device()) if stream is None else stream.cuda_stream
+    _lib.check(_lib.lib().srt_csr_spmm(m, k, n, ci.numel(), rp.data_ptr(), ci.data_ptr(), rp.element_size(),
+                                       vals.data_ptr(), B.data_ptr(), B.stride(0), C.data_ptr(), C.stride(0),
+                                       int(n_tile), s))
     return C
 
 

@@ -17,6 +17,11 @@ def stream_handle(stream: Optional[torch.cuda.Stream] = None) -> ct.c_void_p:
     return ct.c_void_p(s.cuda_stream)
 
 
+def current_raw_stream(device_index: int) -> int:
+    """hipStream_t of the device's current stream, without the Stream object."""
+    return torch._C._cuda_getCurrentRawStream(device_index)
+
+
 def require_cuda_f32(t: torch.Tensor, name: str) -> torch.Tensor:
     if not isinstance(t, torch.Tensor):
         raise TypeError("%s must be a torch.Tensor" % name)

@@ -23,7 +23,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .native import ptr, stream_handle
+from .native import current_raw_stream, ptr, stream_handle
 
 DTYPES = {"bf16": _lib.SRT_DT_BF16, "fp8": _lib.SRT_DT_FP8}
 # launch shapes: index -> (N tile, waves per workgroup, panels per wave)
@@ -73,6 +73,9 @@ class PanelPlan:
         self._h = h
         self.device = device
         self._reserved = (0, 1)
+        self._lib = _lib.lib()
+        st = self.stats()
+        self._panels, self._k_blocks = st["num_panels"], st["k_blocks"]
 
     @classmethod
     def from_csr(cls, csr: torch.Tensor, dtype: str = "bf16") -> "PanelPlan":
@@ -101,8 +104,11 @@ class PanelPlan:
         else:
             out = torch.empty((cols, ldk), dtype=torch.uint8, device=B.device)
             scales = torch.empty(cols, dtype=torch.float32, device=B.device)
-        _lib.call("srt_mfma_convert_b", DTYPES[self.dtype], rows, cols, ptr(B), B.stride(0), ptr(out),
-                  out.stride(0), ptr(scales), stream_handle(stream))
+        s = current_raw_stream(torch.cuda.current_device()) if stream is None else stream.cuda_stream
+        rc = self._lib.srt_mfma_convert_b(DTYPES[self.dtype], rows, cols, B.data_ptr(), B.stride(0), out.data_ptr(), ldk,
+                                          None if scales is None else scales.data_ptr(), s)
+        if rc:
+            _lib.check(rc)
         return out, scales
 
     def reserve(self, n_max: int, ksplit_max: int) -> None:
@@ -121,14 +127,18 @@ class PanelPlan:
         n = Bq.shape[0] if n is None else int(n)
         if Bq.shape[1] < -(-self.k // 32) * 32 or C.shape[0] < self.m or C.shape[1] < n or Bq.shape[0] < n:
             raise ValueError("shape mismatch")
-        st = self.stats()
-        dshape, dks = default_launch(st["num_panels"], st["k_blocks"], n)
-        shape = dshape if shape is None else shape
-        ksplit = dks if ksplit is None else ksplit
+        if shape is None or ksplit is None:
+            dshape, dks = default_launch(self._panels, self._k_blocks, n)
+            shape = dshape if shape is None else shape
+            ksplit = dks if ksplit is None else ksplit
         if ksplit > 1 and (self._reserved[0] < n or self._reserved[1] < ksplit):
             self.reserve(max(n, self._reserved[0]), max(ksplit, self._reserved[1]))
-        _lib.call("srt_mfma_plan_execute", self._h, ptr(C), C.stride(0), ptr(Bq), Bq.stride(0),
-                  ptr(col_scales), n, int(shape), int(ksplit), stream_handle(stream))
+        s = current_raw_stream(torch.cuda.current_device()) if stream is None else stream.cuda_stream
+        rc = self._lib.srt_mfma_plan_execute(self._h, C.data_ptr(), C.stride(0), Bq.data_ptr(), Bq.stride(0),
+                                             None if col_scales is None else col_scales.data_ptr(), n, int(shape),
+                                             int(ksplit), s)
+        if rc:
+            _lib.check(rc)
         return C
 
     # -- inspection -----------------------------------------------------------

@@ -74,6 +74,7 @@ class SlabPool:
     def __init__(self, nbytes: int, device):
         self.nbytes = int(nbytes) >> self.MIN_CLASS << self.MIN_CLASS
         self.buf = torch.empty(self.nbytes, dtype=torch.uint8, device=device)
+        self.floats = self.buf.view(torch.float32)
         self.base = self.buf.data_ptr()
         self.free_lists: Dict[int, List[int]] = {}
         self.top = 0
@@ -111,7 +112,7 @@ class SlabPool:
             self.top = 0
 
     def view(self, off: int, shape, dtype) -> torch.Tensor:
-        n = int(np.prod(shape)) * torch.tensor([], dtype=dtype).element_size()
+        n = math.prod(shape) * dtype.itemsize
         return self.buf[off:off + n].view(dtype).view(*shape)
 
 
@@ -588,13 +589,13 @@ class Server:
         return True
 
     def result_view(self, req: Request) -> torch.Tensor:
-        M = int(self.backend.wM[req.weight])
+        M, N = int(self.backend.wM[req.weight]), req.N
         g = req._group
         if g is not None:   # merged: the request's columns of the block's C
-            c = g.col[id(req)]
-            return self.pool.view(g.off + g.b_bytes, (M, g.ld), torch.float32)[:, c:c + req.N]
-        ld = self.backend.result_ld(req.N)
-        return self.pool.view(req._c_off, (M, ld), torch.float32)[:, :req.N]
+            at, ld = (g.off + g.b_bytes) // 4 + g.col[id(req)], g.ld
+        else:
+            at, ld = req._c_off // 4, self.backend.result_ld(N)
+        return self.pool.floats.as_strided((M, N), (ld, 1), at)
 
     def release(self, req: Request, keep_result: bool = False, stream: Optional[torch.cuda.Stream] = None) -> None:
         """Return the request's memory to the budget.  With keep_result the
@@ -641,9 +642,14 @@ class Server:
         slot = self.slots[slot_index]
         self._fill(slot, batch)
         slot.launch(self.use_graphs)
+        # Every result is copied out before the first block is given back, with
+        # one wait for them all (one each took half the call at 24 requests).
+        with torch.cuda.stream(slot.stream):
+            for r in batch:
+                r.C = self.result_view(r).clone()
         slot.stream.synchronize()
         for r in batch:
-            self.release(r, keep_result=True, stream=slot.stream)
+            self.release(r)
 
     def serve(self, requests: List[Request], keep_results: bool = False) -> Dict[str, float]:
         """Open-loop serving of requests (arrival times in seconds from start).
