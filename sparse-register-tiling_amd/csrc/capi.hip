@@ -1817,10 +1817,20 @@ static int group_bind(srt_group &g, const float *const *B, const int64_t *ldb, f
         V = std::max(V, v);
         least = std::min(least, v);
     }
+    // Problems with the longest workgroups first, so that short ones fill the
+    // end of the launch.
+    std::vector<int> order((size_t)cnt);
+    std::vector<double> length((size_t)cnt, 0.0);
+    for (int i = 0; i < cnt; ++i) {
+        const srt_plan &p = *g.plans[i];
+        order[i] = i;
+        if (p.sch.n_wblocks > 0) length[i] = (double)p.pk.total_cols / p.sch.n_wblocks * (1 + lanes[i]);
+    }
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return length[a] > length[b]; });
     std::vector<ExecProblem> t;
     int64_t total = 0;
     size_t lds = 0;
-    for (int i = 0; i < cnt; ++i) {
+    for (int i : order) {
         const srt_plan &p = *g.plans[i];
         if (n[i] == 0 || p.pk.M == 0 || p.sch.n_wblocks == 0) continue;
         ExecProblem q{};

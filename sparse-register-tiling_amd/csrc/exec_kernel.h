@@ -484,11 +484,18 @@ __global__ void __launch_bounds__(1024)
     exec_grouped_kernel(ConstProblems probs, int nprob, int xcd_remap) {
     extern __shared__ float lds[];
     int b = blockIdx.x;
-    if (xcd_remap) b = xcd_swizzle(b, gridDim.x);
     int lo = 0, hi = nprob - 1;  // last problem with block_begin <= b
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
         if (probs[mid].block_begin <= b) lo = mid; else hi = mid - 1;
+    }
+    // Each problem is dealt to all XCDs, one contiguous run of it to each: over
+    // the whole grid, XCD 0 had the first layers of a network and XCD 7 the
+    // last, whose workgroups are several times longer.
+    if (xcd_remap) {
+        const int begin = probs[lo].block_begin;
+        const int count = (lo + 1 < nprob ? probs[lo + 1].block_begin : (int)gridDim.x) - begin;
+        b = begin + xcd_swizzle(b - begin, count);
     }
     // Each problem runs at its own lane width (at most V): an image of 49
     // pixels keeps 49 of 64 lanes busy at one float per lane, 13 at four, and
