@@ -17,6 +17,7 @@ scales of B, both computed in FP64 on the device:
 from __future__ import annotations
 
 import ctypes as ct
+import functools
 from typing import Dict, Optional, Tuple
 
 import numpy as np
@@ -38,17 +39,53 @@ def _index_tensor(x, device) -> torch.Tensor:
     return t.contiguous()
 
 
-def default_launch(num_panels: int, k_blocks: int, n: int, target_groups: int = 256) -> Tuple[int, int]:
-    """(shape, ksplit) giving about `target_groups` workgroups: 64-column
-    tiles of 8 panels (one per wave, 8 waves), the K range split when panels
-    x tiles are too few."""
-    shape = 6
-    nt, wp, pw = SHAPES[shape]
+# Time model of default_launch, in us: (a launch; a K block of one
+# workgroup's chain, by shape; 10 KB of operand tiles per CU; the second launch of
+# a K split; a million floats of partial tiles).  Least squares over 66 problem
+# sizes (256..4096 rows, 128..4096 deep, 32..2048 columns) times the three shapes
+# times K splits of 1..32.  On average its choice takes 1.03 of the fastest
+# launch's time; 64-column tiles with the K range split up to 256 workgroups,
+# which it replaces, took 1.23 (512 x 512 x 100: 8.1 us, now 6.7; 2048 x 512 x
+# 512: 14.2, now 7.9; 4096 x 1024 x 1024: 19.7 both).
+_LAUNCH_US = 5.39
+_CHAIN_US = ((6, .151), (9, .103), (4, .091))
+_TILE_US, _SPLIT_US, _PARTIAL_US = .101, 1.49, 1.52
+
+
+def _split_limit(num_panels: int, k_blocks: int, n: int, target_groups: int = 256) -> int:
+    """K splits that fill the chip with 64-column tiles of 8 panels: the most a
+    default launch uses, and what it reserves the workspace for, so that the
+    reservation of one call covers every later one that is not wider."""
+    nt, wp, pw = SHAPES[6]
     groups = -(-num_panels // (wp * pw)) * -(-n // nt)
     ks = 1
     while groups * ks * 2 <= target_groups and ks * 2 <= max(1, k_blocks // 4):
         ks *= 2
-    return shape, ks
+    return ks
+
+
+@functools.lru_cache(maxsize=4096)
+def default_launch(num_panels: int, k_blocks: int, n: int, target_groups: int = 256) -> Tuple[int, int]:
+    """(shape, ksplit) of the least modelled time: wide tiles read B and A less
+    often, narrow ones give more workgroups and a shorter chain per K block, a
+    K split shortens the chain for a second launch and the partial tiles.
+    target_groups: workgroups that fill the chip."""
+    limit = _split_limit(num_panels, k_blocks, n, target_groups)
+    best = None
+    for shape, chain in _CHAIN_US:
+        nt, wp, pw = SHAPES[shape]
+        groups = -(-num_panels // (wp * pw)) * -(-n // nt)
+        ks = 1
+        while ks <= limit:
+            steps = -(-k_blocks // ks)
+            t = _LAUNCH_US + chain * steps
+            t += _TILE_US * groups * ks * steps * (wp * pw * 1024 + nt * 64) / target_groups * 1e-4
+            if ks > 1:
+                t += _SPLIT_US + _PARTIAL_US * (ks + 1) * num_panels * 16 * n * 1e-6
+            if best is None or t < best[0]:
+                best = (t, shape, ks)
+            ks *= 2
+    return best[1], best[2]
 
 
 class PanelPlan:
@@ -130,9 +167,14 @@ class PanelPlan:
         if shape is None or ksplit is None:
             dshape, dks = default_launch(self._panels, self._k_blocks, n)
             shape = dshape if shape is None else shape
-            ksplit = dks if ksplit is None else ksplit
-        if ksplit > 1 and (self._reserved[0] < n or self._reserved[1] < ksplit):
-            self.reserve(max(n, self._reserved[0]), max(ksplit, self._reserved[1]))
+            if ksplit is None:
+                ksplit, need = dks, _split_limit(self._panels, self._k_blocks, n)
+            else:
+                need = ksplit
+        else:
+            need = ksplit
+        if need > 1 and (self._reserved[0] < n or self._reserved[1] < need):
+            self.reserve(max(n, self._reserved[0]), max(need, self._reserved[1]))
         s = current_raw_stream(torch.cuda.current_device()) if stream is None else stream.cuda_stream
         rc = self._lib.srt_mfma_plan_execute(self._h, C.data_ptr(), C.stride(0), Bq.data_ptr(), Bq.stride(0),
                                              None if col_scales is None else col_scales.data_ptr(), n, int(shape),

@@ -1,6 +1,7 @@
-"""The sum of a K split over panels.
+"""The panel launch rule and the K split's sum.
 
-The sum of the partial tiles adds them in split order in
+The rule never splits further than its workspace limit and names a launch
+shape that exists.  The sum of the partial tiles adds them in split order in
 16-byte and in 4-byte rows: both give the same bits, at row lengths around a
 block's width and at split counts around the four that are loaded together.
 """
@@ -12,6 +13,16 @@ import pytest
 def pr():
     import importlib
     return importlib.import_module("sparse-register-tiling_amd").precision
+
+
+def test_rule_stays_within_its_workspace(pr):
+    for panels in (0, 1, 3, 16, 63, 64, 255, 4096):
+        for blocks in (0, 1, 4, 5, 31, 128, 1024):
+            for n in (1, 31, 32, 33, 100, 512, 4096, 100000):
+                shape, ks = pr.default_launch(panels, blocks, n)
+                assert shape in pr.SHAPES
+                assert 1 <= ks <= pr._split_limit(panels, blocks, n)
+                assert ks == 1 or ks * 4 <= blocks
 
 
 @pytest.mark.gpu
