@@ -1,0 +1,47 @@
+"""Dense panels of a hybrid plan: output tiles and K splits.
+
+Every launch the rule can take covers all rows, columns and K ranges: sizes
+around the tiles' edges (32, 64, 128 rows; 64, 128 columns; 64 deep), widths
+that are no multiple of 4 (the narrow B loads), and products from one tile to
+several rounds of the chip.  K chains of fp32 products and their sums: within
+(K + 40) * 2^-24 * |A| |B| of the float64 product, and equal bits on a repeat.
+"""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def srt():
+    import importlib
+    return importlib.import_module("sparse-register-tiling_amd")
+
+
+@pytest.mark.parametrize("mkn", [(16, 64, 16), (33, 65, 64), (31, 700, 65), (96, 130, 127), (64, 64, 128), (129, 513, 129),
+                                 (512, 512, 128), (512, 2048, 256), (300, 1500, 333), (256, 4096, 512), (1024, 1024, 512),
+                                 (4096, 256, 512), (2048, 512, 100), (4096, 4096, 64), (2064, 192, 1030),
+                                 (1024, 4096, 512)])
+def test_tiles_and_splits(srt, mkn):
+    import torch
+    M, K, N = mkn
+    print("dense tiles", mkn, flush=True)
+    g = torch.Generator().manual_seed(M + K + N)
+    A = torch.randn(M, K, generator=g) * (torch.rand(M, K, generator=g) < 0.5)
+    B = torch.randn(K, N, generator=g).cuda()
+    plan = srt.MatMulSpecialized.from_csr(A.to_sparse_csr().cuda(), N, mapping_id=srt.named_mapping(4, "orig"),
+                                          dense_threshold=0.2)
+    out = torch.full((M, N), float("nan"), device="cuda")
+    plan(out, B)
+    again = torch.full((M, N), float("nan"), device="cuda")
+    plan(again, B)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
+    Ad = A.cuda().double()
+    err = (out.double() - Ad @ B.double()).abs()
+    bound = (Ad.abs() @ B.double().abs()) * (K + 40) * 2.0 ** -24
+    assert bool((err <= bound + 1e-30).all())
+    # a narrower product through the same plan: another grid, the same workspace
+    n = max(1, N // 3)
+    part = torch.full((M, n), float("nan"), device="cuda")
+    plan(part, B[:, :n].contiguous())
+    assert bool(((part.double() - Ad @ B[:, :n].double()).abs() <= bound[:, :n] + 1e-30).all())
