@@ -602,9 +602,15 @@ static int cu_count() {
 // bytes in fewer batches.  Both sides at 16 waves, 8-row "orig": 4096 x 1024
 // at 90 % x 200 runs 19.5 us at V = 4 (512 workgroups) and 31.6 at V = 1;
 // 1000 x 777 at 80 % x 200 runs 12.4 at V = 1 and 16.1 at V = 4 (125).  Two
-// floats pay only with half a round more.  Waves: 16 beat 8 at 62 of 72
-// sizes (M 256-4096, K 512-4096, N 8-1024), by a tenth at the middle one,
-// and lose at most 6 %.
+// floats pay only with half a round more.
+//
+// Waves: 8 at every size (plans of one group have to agree).  16 are about a
+// twentieth faster on small products and up to a half slower on large ones
+// (996 x 2291 x 2344, 4-row "orig": 1.29 of the time of 8).  Chunks: with more
+// than four N tiles workgroups are many, and half as many columns a chunk even
+// out the CUs: 0.89 of the time on average over 34 products of 5..13 tiles
+// (0.72 to 1.08); with fewer tiles a panel's extra chunks only open a second
+// round (1.10 over 26).
 static void realise_config(srt_tile_config &c, int P, int M_r, int K, int K_tile, int64_t total_cols, int n) {
     if (c.vec_width != 1 && c.vec_width != 2 && c.vec_width != 4) {
         const int64_t cus = cu_count();
@@ -612,7 +618,8 @@ static void realise_config(srt_tile_config &c, int P, int M_r, int K, int K_tile
                       : n > 64 && 2 * (int64_t)P * ((n + 127) / 128) >= 3 * cus  ? 2
                                                                                  : 1;
     }
-    if (c.waves_per_block < 1 || c.waves_per_block > kMaxWaves) c.waves_per_block = 16;
+    const bool own = c.waves_per_block < 1 || c.waves_per_block > kMaxWaves;
+    if (own) c.waves_per_block = 8;
     if (c.nsplit < 1 || c.nsplit > c.waves_per_block) c.nsplit = c.waves_per_block;
     // B path: global-memory rows unless the LDS tile is asked for and its
     // narrowest form (V = 1) fits (measured faster on the pruned-FFN shapes).
@@ -633,6 +640,7 @@ static void realise_config(srt_tile_config &c, int P, int M_r, int K, int K_tile
         const int64_t n_tiles = (n + 64 * c.vec_width - 1) / (64 * c.vec_width);
         const int64_t target_waves = 4096;
         c.chunk_cols = (int)std::max<int64_t>(8, (total_cols * n_tiles + target_waves - 1) / target_waves);
+        if (own && n_tiles > 4 && c.chunk_cols > 60) c.chunk_cols = std::max(60, c.chunk_cols / 2);
     }
     if (c.xcd_remap != 0 && c.xcd_remap != 1) c.xcd_remap = 1;
     if (!pow2_upto8(c.unroll)) c.unroll = 4;
