@@ -516,6 +516,8 @@ def bench_hybrid(args):
         t_plain = at.time_graph(lambda: plain(C, Bd), reps=30)
         cfg = plain.get_config()
         mp = plain.mapping
+        if cfg.b_staging == 3:  # as autotune.tuned_hybrid
+            cfg, mp = None, srt.named_mapping(4, "orig")
         plain.close()
         A_dev = torch.from_numpy(A).cuda()
         t_dense = at.time_graph(lambda: torch.matmul(A_dev, Bd, out=C), reps=30)

@@ -505,8 +505,8 @@ def tuned_hybrid(csr: torch.Tensor, N: int, thresholds: Sequence[float] = HYBRID
                  path: str = SHIPPED) -> Tuple[MatMulSpecialized, Dict[str, object]]:
     """The fastest of the tuned plain plan and its hybrids (16-row panels at
     least `threshold` dense on FP32 matrix cores, the rest register-tiled
-    with the plain plan's mapping and configuration), graph-timed on the
-    device at width N.  The reference fixes its dense-tile threshold at 0.30
+    with the plain plan's mapping and configuration, the default one where
+    that streams), graph-timed on the device at width N.  The reference fixes its dense-tile threshold at 0.30
     (sbench/padding_reordering.py:36); here each threshold that yields a
     different set of dense panels is timed and the measurement decides.
     Returns the plan and a report {"plain_s", "choice": threshold or None,
@@ -521,6 +521,11 @@ def tuned_hybrid(csr: torch.Tensor, N: int, thresholds: Sequence[float] = HYBRID
     best_s = time_graph(lambda: best(C, B), reps=reps)
     report: Dict[str, object] = {"plain_s": best_s, "choice": None, "candidates": []}
     cfg, mapping = best.get_config(), best.mapping
+    if cfg.b_staging == 3:
+        # the few rows a hybrid leaves would stream all of B: the gather
+        # default instead (4096 x 1024 x 512: 71.9 us with 3 of 256 panels
+        # left to streaming, 55.9 with 7 left to the gather)
+        cfg, mapping = None, named_mapping(4, "orig")
     seen = set()
     for tau in sorted(thresholds):
         hp = MatMulSpecialized.from_csr(csr, N, mapping_id=mapping, tile_config=cfg, dense_threshold=tau)

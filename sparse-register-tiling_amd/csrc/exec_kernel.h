@@ -500,7 +500,8 @@ __global__ void __launch_bounds__(1024)
     // Each problem runs at its own lane width (at most V): an image of 49
     // pixels keeps 49 of 64 lanes busy at one float per lane, 13 at four, and
     // does not hold the wide problems to its width.  16 layers of a network,
-    // one of them of 49 columns: 97.5 us at the narrowest's width, 58.7 so.
+    // one of them of 49 columns: 97.5 us at the narrowest's width, 58.7 so
+    // (44.9 with the order of workgroups above).
     const int lanes = probs[lo].lanes;
     if constexpr (V >= 4)
         if (lanes == 4) return grouped_body<MR, 4, U, STAGE, D>(lds, probs, lo, b);

@@ -24,12 +24,15 @@
 // identity: value -0.0 against a row of +0.0 leaves every accumulator, signed
 // zero and NaN included, as it is.
 //
-// Measured (4096 x 1024 at 80 % times 1024 x 2048): 110.8 us, the gather
-// executor 168.2 (31.0 and 20.4 TFLOP/s).  What bounds it is the scalar
-// unit's supply of entries, about 1000 clocks per block of a wave with the
-// chip full: LDS reads alone would take 51 us, the multiply-adds 22.  Entries
-// brought through vector registers instead (DPP broadcasts 139 us, readlane
-// 280 us) and blocks fetched into the L2 a tile ahead (142 us) were slower.
+// Measured (4096 x 1024 at 80 % times 1024 x 2048): 110.7 us, the gather
+// executor 168.7 (31.1 and 20.4 TFLOP/s).  What bounds it is instruction
+// issue: per entry a wave issues V multiply-adds, an LDS read and about one
+// scalar instruction, 4.3 and 4.4 clocks of a SIMD each (8 multiply-adds and 8
+// scalar instructions together take 44 clocks), and waits for its scalar
+// loads; LDS reads alone would take 51 us, the multiply-adds 22.  Half the
+// bytes per entry (16-bit row words) took 138 us, since unpacking costs scalar
+// instructions; entries through vector registers (DPP broadcasts 139 us,
+// readlane 280) and blocks fetched into the L2 a tile ahead (142) were slower.
 // Staging costs a workgroup the L2's 64 bytes per clock and CU, shared by its
 // W * R rows: with few rows (little work) the gather executor is the faster.
 #include <hip/hip_runtime.h>
