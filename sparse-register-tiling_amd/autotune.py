@@ -470,11 +470,17 @@ def streamed_launch(M: int, K: int, nnz: int, N: int) -> Tuple[int, int, float]:
 
 def gather_seconds(M: int, K: int, nnz: int, N: int) -> float:
     """Estimated seconds of the gather executor with the 4-row "orig" mapping
-    on the same sizes: 4 us and 0.16 us per 10^6 products, times the packed
-    columns per nonzero of a 4-row panel (one B row gathered for each)."""
+    on the same sizes: 4 us, 3 ns per B row (a panel's chain) and 0.2 us per
+    10^6 products, times the packed columns per nonzero of a 4-row panel (one
+    B row gathered for each); below 256 columns whole waves of 64.  On 60
+    drawn sizes (M 256-4096, K 128-4096, N 1-4096, 66-97 % sparse) the lower
+    estimate takes 1.004 of the faster executor's time on average and 1.11 at
+    worst (1.013 and 1.53 on 60 others); without the chain and at 0.16 us 1.03 and
+    1.60."""
     d = nnz / float(max(1, M * K))
     share = (1.0 - (1.0 - d) ** 4) / (4.0 * d) if d > 0 else 1.0
-    return 4e-6 + 0.16e-12 * share * nnz * N
+    width = N if N >= 256 else -(-N // 64) * 64
+    return 4e-6 + 3e-9 * K + 0.2e-12 * share * nnz * width
 
 
 def tuned_plan(csr: torch.Tensor, N: int, path: str = SHIPPED) -> MatMulSpecialized:
