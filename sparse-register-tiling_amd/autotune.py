@@ -475,8 +475,8 @@ def gather_seconds(M: int, K: int, nnz: int, N: int) -> float:
     B row gathered for each); below 256 columns whole waves of 64.  On 60
     drawn sizes (M 256-4096, K 128-4096, N 1-4096, 66-97 % sparse) the lower
     estimate takes 1.004 of the faster executor's time on average and 1.11 at
-    worst (1.013 and 1.53 on 60 others); without the chain and at 0.16 us 1.03 and
-    1.60."""
+    worst, on 60 others 1.013 and 1.53; without the chain and at 0.16 us it
+    took 1.03 and 1.60 on the first."""
     d = nnz / float(max(1, M * K))
     share = (1.0 - (1.0 - d) ** 4) / (4.0 * d) if d > 0 else 1.0
     width = N if N >= 256 else -(-N // 64) * 64
