@@ -495,7 +495,10 @@ def tuned_plan(csr: torch.Tensor, N: int, path: str = SHIPPED) -> MatMulSpeciali
     if not recs:
         nnz = csr.values().numel()
         V, R, seconds = streamed_launch(M, K, nnz, N)
-        if seconds < gather_seconds(M, K, nnz, N):
+        # Fewer than 32 columns: streaming gains a tenth at best, and loses a
+        # fifth where its tiles are short of rows (3835 x 2508 at 70 % x 3:
+        # 54.9 us, 45.5 gathered).
+        if N >= 32 and seconds < gather_seconds(M, K, nnz, N):
             return MatMulSpecialized.from_csr(csr, N, mapping_id=named_mapping(1, "identity"),
                                               tile_config=TileConfig(b_staging=3, vec_width=V, waves_per_block=16,
                                                                      chunk_cols=R))
