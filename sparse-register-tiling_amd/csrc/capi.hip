@@ -1355,7 +1355,8 @@ static int ensure_gather(const srt_plan *cp) {
     if (p->sch.desc) return SRT_OK;
     srt_tile_config c = p->cfg_user;
     c.b_staging = 2;
-    c.chunk_cols = c.nsplit = 0;
+    c.chunk_cols = 0;
+    c.nsplit = 1;  // one chain per row: the bits of the streamed launch
     const int n = std::max(p->n_max, 1);
     realise_config(c, p->pk.P, p->pk.M_r, p->pk.K, p->pk.K_c, p->pk.total_cols, n);
     Schedule sch;

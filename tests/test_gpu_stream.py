@@ -101,7 +101,8 @@ def test_other_widths_groups_and_graphs(srt, oracle):
     C.zero_()
     grp()
     torch.cuda.synchronize()
-    assert np.allclose(C.cpu().numpy(), ref, rtol=0, atol=1e-4) and torch.equal(C, C2)
+    _same(C.cpu().numpy(), ref)  # the bits of its own launch
+    assert torch.equal(C, C2)
     grp.close()
     rp, ci, v = srt.workloads.to_csr(A)
     h = srt.MatMulSpecialized(200, 150, 300, torch.from_numpy(v), torch.from_numpy(rp), torch.from_numpy(ci),
