@@ -1366,6 +1366,14 @@ static int ensure_gather(const srt_plan *cp) {
     return SRT_OK;
 }
 
+// Panels the register-tiled part of a plan runs (a hybrid's dense panels are
+// not among them): what its launch geometry is chosen for.  704 x 992 x 320
+// with 36 of 44 panels dense: 26.4 us at the lane width of 176 panels, 22.3 at
+// that of the 32 left; 2279 x 3952 x 166, 130 of 143: 102.5 and 81.0.
+static int active_panels(const Packed &pk) {
+    return pk.P - (int)std::count(pk.h_skip.begin(), pk.h_skip.end(), 1);
+}
+
 // Panel ranges of the matrix-core executor for B width n: R contiguous
 // ranges balanced by packed columns (+4 per panel for its C rows), R x
 // (64-column slices) = one round of 256 CUs; the ranges of a width used
@@ -1603,6 +1611,8 @@ int srt_plan_create_hybrid(int m, int k, int n, const float *Lx, const void *Lp,
         } else {
             Schedule first = std::move(plan->sch);
             plan->sch = Schedule();
+            plan->cfg = plan->cfg_user;
+            realise_config(plan->cfg, active_panels(pk), pk.M_r, pk.K, pk.K_c, pk.total_cols, std::max(n, 1));
             const int rc = build_schedule(pk, plan->cfg, plan->exec, config_tiles(plan->cfg, std::max(n, 1)),
                                           plan->sch, plan->retired, plan->cfg, s);
             first.release();
@@ -1657,7 +1667,7 @@ int srt_plan_allocate_executor(srt_plan *p, int n) {
         p->cfg = c;
         return SRT_OK;
     }
-    realise_config(c, p->pk.P, p->pk.M_r, p->pk.K, p->pk.K_c, p->pk.total_cols, std::max(n, 1));
+    realise_config(c, active_panels(p->pk), p->pk.M_r, p->pk.K, p->pk.K_c, p->pk.total_cols, std::max(n, 1));
     const int tiles = config_tiles(c, std::max(n, 1));
     srt_tile_config sch_cfg = p->cfg;
     SRT_TRY(switch_schedule(p->pk, c, tiles, p->exec, p->sch, sch_cfg, p->retired, nullptr));
