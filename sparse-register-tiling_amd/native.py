@@ -8,7 +8,7 @@ from typing import Optional, Sequence, Union
 import torch
 
 from . import _lib
-from .mapping import (MAPPINGS_DIR, STRATEGY_M_R, Mapping, find_mapping, named_mapping, read_mapping_file,
+from .mapping import (MAPPINGS_DIR, NAMED_IDS, STRATEGY_M_R, Mapping, find_mapping, named_mapping, read_mapping_file,
                       strategy_for)
 
 
@@ -108,6 +108,9 @@ def resolve_mapping(mapping: Union[str, Mapping, NativeMapping], M_r: Optional[i
     if M_r is not None:
         return NativeMapping.from_mapping(named_mapping(M_r, mapping, search_dirs))
     for mr in sorted(set(STRATEGY_M_R.values())):
+        # a bare name never means one row per panel: "identity" is the 2-row one
+        if mr == 1 and mapping in NAMED_IDS[1]:
+            continue
         if strategy_for(mr, mapping) is not None:
             return NativeMapping.from_mapping(named_mapping(mr, mapping, search_dirs))
     return NativeMapping.from_id(mapping, search_dirs)

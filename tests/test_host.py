@@ -307,3 +307,14 @@ def test_counter_means_reads_rocprof_csv(srt, tmp_path):
     assert m["exec_kernel<4>"] == {"FETCH_SIZE": 5000.0, "WRITE_SIZE": 2048.0}
     assert m["elementwise_kernel"] == {"FETCH_SIZE": 262144.0}
     assert at._counter_means(str(tmp_path), last=1)["exec_kernel<4>"]["FETCH_SIZE"] == 6000.0
+
+
+def test_bare_names_mean_the_panel_heights_they_meant(srt):
+    """A name without M_r is the lowest of the reference's panel heights that
+    has it: "identity" is the 2-row mapping.  The 1-row mapping of the streamed
+    executor answers to its id, and to its name with M_r = 1."""
+    assert srt.resolve_mapping("identity").M_r == 2
+    assert srt.get_executor_id("identity") == srt.resolve_mapping("4af51").executor_id()
+    assert srt.resolve_mapping("orig").M_r == 4
+    assert srt.resolve_mapping("2b3d8").M_r == 1
+    assert srt.resolve_mapping("identity", M_r=1).M_r == 1
