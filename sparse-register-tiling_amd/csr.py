@@ -23,8 +23,10 @@ def _parts(csr: torch.Tensor):
     if csr.dim() != 2:
         raise ValueError("expected a 2-D CSR matrix")
     rp, ci, vals = csr.crow_indices(), csr.col_indices(), csr.values()
-    if not (csr.is_cuda and vals.dtype is torch.float32 and ci.dtype is rp.dtype and rp.is_contiguous()
-            and ci.is_contiguous() and vals.is_contiguous()):
+    # As it is only where the kernel runs: another GPU's memory may not be
+    # readable from here.
+    if not (rp.is_cuda and rp.get_device() == torch.cuda.current_device() and vals.dtype is torch.float32
+            and ci.dtype is rp.dtype and rp.is_contiguous() and ci.is_contiguous() and vals.is_contiguous()):
         rp = rp.cuda().contiguous()
         ci = ci.cuda().contiguous()
         if ci.dtype != rp.dtype:
