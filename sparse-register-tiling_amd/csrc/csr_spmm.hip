@@ -65,11 +65,13 @@ __global__ void __launch_bounds__(256)
     end = end > nnz ? nnz : (end < q ? q : end);
     // Lane l holds entry l of 64: B row offset (bytes, or rows when BIG) and
     // value; a lane without one holds row 0 and is not multiplied.
+    // Ends are compared as differences: within 64 entries of the largest I a
+    // sum past the end wraps to an index below the arrays.
     I c = -1;
     float a = 0.0f;
     auto fetch = [&](I at) {
         c = -1;
-        if (at + lane < end) {
+        if (lane < end - at) {
             c = colind[at + lane];
             a = vals[at + lane];
         }
@@ -107,7 +109,7 @@ __global__ void __launch_bounds__(256)
         take();
         load(r0, 0);
     }
-    for (; q + 64 < end; q += 64) {
+    for (; end - q > 64; q += 64) {
         fetch(q + 64);
         load(r1, 16);
         add(r0, val, 0, kBatch);

@@ -110,3 +110,30 @@ def test_operand_preparation(srt, K, N):
     q = torch.zeros((N, ldk), dtype=torch.uint8, device="cuda")
     q[:, :K] = (B.double() / scale.double()).float().t().contiguous().to(torch.float8_e4m3fn).view(torch.uint8)
     assert torch.equal(Bq, q)
+
+
+@pytest.mark.parametrize("N", [3, 70, 130])
+def test_csr_rows_at_the_end_of_the_index_range(srt, oracle, N):
+    """int32 indices and 2^31 - 1 stored entries: the last rows end where a sum
+    past the end does not fit the index type.  Only those rows are in the
+    product, and only their entries of the arrays are written."""
+    import torch
+    _, cb = oracle
+    nnz, K, lengths = 2 ** 31 - 1, 200, [1, 64, 65, 130, 40, 0, 20]
+    if torch.cuda.mem_get_info()[0] < 24 << 30:
+        pytest.skip("needs 24 GiB of device memory")
+    print("csr at 2^31 - 1 entries", N, flush=True)
+    rng = np.random.default_rng(N)
+    used = sum(lengths)
+    ci = np.concatenate([rng.permutation(K)[:l] for l in lengths]).astype(np.int32)
+    v = rng.standard_normal(used).astype(np.float32)
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    rp = (nnz - used + np.concatenate([[0], np.cumsum(lengths)])).astype(np.int32)
+    cols, vals = torch.empty(nnz, dtype=torch.int32, device="cuda"), torch.empty(nnz, device="cuda")
+    cols[-used:], vals[-used:] = torch.from_numpy(ci).cuda(), torch.from_numpy(v).cuda()
+    shape = torch.sparse_csr_tensor(torch.zeros(len(lengths) + 1, dtype=torch.int32), torch.zeros(0, dtype=torch.int32),
+                                    torch.zeros(0), size=(len(lengths), K))
+    C = srt.csr.spmm(shape, torch.from_numpy(B).cuda(), _parts_cache=(torch.from_numpy(rp).cuda(), cols, vals))
+    torch.cuda.synchronize()
+    ref = cb.csr_exec((rp - rp[0]).astype(np.int64), ci.astype(np.int64), v, len(lengths), B)
+    assert np.array_equal(C.cpu().numpy().view(np.uint32), ref.view(np.uint32))
