@@ -396,7 +396,9 @@ typedef struct srt_mfma_stats {
 int srt_mfma_plan_create(int m, int k, const float *Lx, const void *Lp, const void *Li, int index_bytes,
                          int dtype, srt_stream_t stream, srt_mfma_plan **out);
 /* Workspace for K-split launches: up to ksplit_max partial tiles of m x n_max.
- * Allocates; call it before capturing launches in a graph. */
+ * Allocates; call it before capturing launches in a graph.  A workspace that
+ * is outgrown stays alive until the plan is destroyed: graphs that captured
+ * launches with it replay unchanged. */
 int srt_mfma_plan_reserve(srt_mfma_plan *p, int n_max, int ksplit_max);
 /* fp32 B (rows = K x cols = N, row-major, ldb) -> Bt: N x ld_out in BF16 or
  * e4m3, k contiguous (the MFMA B operand order), ld_out >= K rounded up to 32,

@@ -45,6 +45,7 @@ struct srt_mfma_plan {
     float *rscale = nullptr;
     float *work = nullptr;
     size_t work_floats = 0;
+    std::vector<float *> retired_work;  // outgrown ones, alive for graphs that captured them
     ~srt_mfma_plan() {
         (void)hipFree(present);
         (void)hipFree(slot);
@@ -52,6 +53,7 @@ struct srt_mfma_plan {
         (void)hipFree(blocks);
         (void)hipFree(rscale);
         (void)hipFree(work);
+        for (float *w : retired_work) (void)hipFree(w);
     }
 };
 
@@ -179,11 +181,13 @@ int srt_mfma_plan_reserve(srt_mfma_plan *p, int n_max, int ksplit_max) {
     if (n_max < 0 || ksplit_max < 1) return fail(SRT_ERR_INVALID, "bad reservation");
     const size_t need = ksplit_max > 1 ? (size_t)ksplit_max * p->M * n_max : 0;
     if (need <= p->work_floats) return SRT_OK;
-    (void)hipFree(p->work);
-    p->work = nullptr;
-    p->work_floats = 0;
-    MF_TRY(dalloc(&p->work, need));
-    p->work_floats = need;
+    // At least twice the outgrown one: all that are kept hold less than the last.
+    const size_t floats = std::max(need, 2 * p->work_floats);
+    float *w = nullptr;
+    MF_TRY(dalloc(&w, floats));
+    if (p->work) p->retired_work.push_back(p->work);
+    p->work = w;
+    p->work_floats = floats;
     return SRT_OK;
 }
 

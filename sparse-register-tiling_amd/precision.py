@@ -54,8 +54,7 @@ _TILE_US, _SPLIT_US, _PARTIAL_US = .101, 1.49, 1.52
 
 def _split_limit(num_panels: int, k_blocks: int, n: int, target_groups: int = 256) -> int:
     """K splits that fill the chip with 64-column tiles of 8 panels: the most a
-    default launch uses, and what it reserves the workspace for, so that the
-    reservation of one call covers every later one that is not wider."""
+    default launch uses.  The fewer columns, the more splits."""
     nt, wp, pw = SHAPES[6]
     groups = -(-num_panels // (wp * pw)) * -(-n // nt)
     ks = 1
@@ -88,6 +87,21 @@ def default_launch(num_panels: int, k_blocks: int, n: int, target_groups: int = 
     return best[1], best[2]
 
 
+@functools.lru_cache(maxsize=4096)
+def split_reservation(num_panels: int, k_blocks: int) -> Tuple[int, int]:
+    """(columns, K splits) of the largest workspace a default launch of any
+    width can need: one reservation covers them all, at most 256 tiles of
+    128 x 64 floats (8 MiB).  (0, 1) where no width is split."""
+    best, columns = (0, 1), SHAPES[6][0]
+    while True:
+        ks = _split_limit(num_panels, k_blocks, columns)
+        if ks == 1:
+            return best
+        if ks * columns > best[0] * best[1]:
+            best = (columns, ks)
+        columns += SHAPES[6][0]
+
+
 class PanelPlan:
     """Packed 16-row panels of A on the device for BF16 or FP8 MFMA."""
 
@@ -109,7 +123,7 @@ class PanelPlan:
                   Lp_t.element_size(), DTYPES[dtype], stream_handle(stream), ct.byref(h))
         self._h = h
         self.device = device
-        self._reserved = (0, 1)
+        self._reserved = 0  # floats of the K-split workspace
         self._lib = _lib.lib()
         st = self.stats()
         self._panels, self._k_blocks = st["num_panels"], st["k_blocks"]
@@ -149,9 +163,11 @@ class PanelPlan:
         return out, scales
 
     def reserve(self, n_max: int, ksplit_max: int) -> None:
-        """Workspace for K-split launches (allocates; do it before graph capture)."""
+        """Workspace for K-split launches (allocates; do it before graph capture).
+        A smaller one stays alive for the graphs that captured it."""
         _lib.call("srt_mfma_plan_reserve", self._h, int(n_max), int(ksplit_max))
-        self._reserved = (max(self._reserved[0], n_max), max(self._reserved[1], ksplit_max))
+        if ksplit_max > 1:
+            self._reserved = max(self._reserved, int(ksplit_max) * self.m * int(n_max))
 
     def __call__(self, C: torch.Tensor, Bq: torch.Tensor, col_scales: Optional[torch.Tensor] = None,
                  n: Optional[int] = None, shape: Optional[int] = None, ksplit: Optional[int] = None,
@@ -164,17 +180,16 @@ class PanelPlan:
         n = Bq.shape[0] if n is None else int(n)
         if Bq.shape[1] < -(-self.k // 32) * 32 or C.shape[0] < self.m or C.shape[1] < n or Bq.shape[0] < n:
             raise ValueError("shape mismatch")
-        if shape is None or ksplit is None:
+        chosen = ksplit is None
+        if shape is None or chosen:
             dshape, dks = default_launch(self._panels, self._k_blocks, n)
             shape = dshape if shape is None else shape
-            if ksplit is None:
-                ksplit, need = dks, _split_limit(self._panels, self._k_blocks, n)
+            ksplit = dks if chosen else ksplit
+        if ksplit > 1 and ksplit * self.m * n > self._reserved:
+            if chosen:  # for every width at once
+                self.reserve(*split_reservation(self._panels, self._k_blocks))
             else:
-                need = ksplit
-        else:
-            need = ksplit
-        if need > 1 and (self._reserved[0] < n or self._reserved[1] < need):
-            self.reserve(max(n, self._reserved[0]), max(need, self._reserved[1]))
+                self.reserve(n, ksplit)
         s = current_raw_stream(torch.cuda.current_device()) if stream is None else stream.cuda_stream
         rc = self._lib.srt_mfma_plan_execute(self._h, C.data_ptr(), C.stride(0), Bq.data_ptr(), Bq.stride(0),
                                              None if col_scales is None else col_scales.data_ptr(), n, int(shape),
