@@ -1658,6 +1658,13 @@ int srt_plan_allocate_executor(srt_plan *p, int n) {
         realise_stream(c, p->pk.M, p->pk.K, p->pk.K_c, p->pk.total_cols, std::max(n, 1));
         if (c.vec_width == p->stream.V && c.waves_per_block == p->stream.waves && c.chunk_cols == p->stream.R)
             return SRT_OK;
+        // A schedule of an earlier width comes back (36 launch shapes at most).
+        for (StreamSched &r : p->retired_streams)
+            if (c.vec_width == r.V && c.waves_per_block == r.waves && c.chunk_cols == r.R) {
+                std::swap(r, p->stream);
+                p->cfg = c;
+                return SRT_OK;
+            }
         if (!p->pk.cols && p->pk.total_cols)
             return fail(SRT_ERR_INVALID, "the plan's column indices were released: its schedule cannot change");
         StreamSched st;

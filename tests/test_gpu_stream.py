@@ -128,3 +128,26 @@ def test_rule_takes_streams_for_much_work(srt):
     at = srt.autotune
     assert at.streamed_launch(4096, 1024, 838860, 2048)[2] < at.gather_seconds(4096, 1024, 838860, 2048)
     assert at.streamed_launch(512, 512, 13107, 8)[2] > at.gather_seconds(512, 512, 13107, 8)
+
+
+def test_alternating_widths_reuse_their_schedules(srt, oracle):
+    """allocate_executor between two widths builds each launch shape once."""
+    import torch
+    _, cb = oracle
+    A = srt.workloads.magnitude_pruned(1024, 1024, 0.5, seed=6)
+    B = srt.workloads.dense_b(1024, 64, seed=7)
+    ref = _chain(srt, cb, A, B)
+    plan = _plan(srt, torch, A, 64)
+    Bt, C = torch.from_numpy(B).cuda(), torch.empty((1024, 64), device="cuda")
+    shapes, free = set(), None
+    for i in range(24):
+        plan.allocate_executor(2048 if i % 2 == 0 else 64)
+        c = plan.get_config()
+        shapes.add((c.vec_width, c.chunk_cols))
+        plan(C, Bt)
+        torch.cuda.synchronize()
+        _same(C.cpu().numpy(), ref)
+        if i == 3:
+            free = torch.cuda.mem_get_info()[0]
+    assert len(shapes) == 2
+    assert torch.cuda.mem_get_info()[0] >= free  # a further copy of the entries is 5 MB
