@@ -553,7 +553,10 @@ static int log2_small(int v) { return v >= 8 ? 3 : v >= 4 ? 2 : v >= 2 ? 1 : 0; 
 static bool pow2_upto8(int v) { return v == 1 || v == 2 || v == 4 || v == 8; }
 
 static constexpr int kMaxWaves = 16;        // wave slots per workgroup (launch bound 1024)
-static constexpr size_t kMaxLdsL2 = 131072;  // reduction LDS of the global-memory B path: 16 waves of 8 rows, V = 4
+// Reduction LDS of the global-memory B path: two workgroups of 16 waves share a
+// CU.  16 waves of 8-row panels run at two floats per lane; four (128 KiB)
+// took 0.53 to 1.37 of the time over 30 sizes, the small ones the longer.
+static constexpr size_t kMaxLdsL2 = 65536;
 
 static size_t reduce_lds(int waves, int M_r, int V) { return (size_t)waves * M_r * V * 64 * sizeof(float); }
 static size_t tile_lds(int K, int V) { return (size_t)K * 64 * V * sizeof(float); }

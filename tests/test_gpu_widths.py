@@ -137,3 +137,24 @@ def test_csr_rows_at_the_end_of_the_index_range(srt, oracle, N):
     torch.cuda.synchronize()
     ref = cb.csr_exec((rp - rp[0]).astype(np.int64), ci.astype(np.int64), v, len(lengths), B)
     assert np.array_equal(C.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+
+
+def test_lane_width_of_many_waves_stays_within_its_lds(srt):
+    """16 waves of 8-row panels reduce in 64 KiB: two floats per lane, whatever
+    the width asked for, and a problem table entry of four is refused."""
+    import ctypes as ct
+
+    import torch
+    A = srt.workloads.magnitude_pruned(256, 300, 0.8, seed=1)
+    rp, ci, v = srt.workloads.to_csr(A)
+    plan = srt.MatMulSpecialized(256, 300, 512, torch.from_numpy(v), torch.from_numpy(rp), torch.from_numpy(ci),
+                                 tile_config=srt.TileConfig(vec_width=4, waves_per_block=16, nsplit=16, unroll=4),
+                                 mapping_id=srt.named_mapping(8, "orig"))
+    assert plan.get_config().vec_width == 2
+    assert max(plan.split_counts()) > 1  # the plan reduces
+    B, C = torch.zeros((300, 512), device="cuda"), torch.zeros((256, 512), device="cuda")
+    out = (ct.c_uint8 * 128)()
+    fill = srt._lib.lib().srt_exec_problem_fill
+    args = lambda V: (plan._h, B.data_ptr(), 512, C.data_ptr(), 512, 512, V, 0, ct.byref(out))
+    assert fill(*args(2)) == 0
+    assert fill(*args(4)) == srt._lib.SRT_ERR_UNSUPPORTED
