@@ -595,17 +595,33 @@ static int cu_count() {
     return cached[dev];
 }
 
+// Default floats per lane of a gather launch (8 waves).  A wide lane takes fewer
+// batches for the same bytes, so it wins where workgroups are many (more than
+// 12 panels x 64-column slices per CU) or the L2 serves most gathers: a slice is
+// walked by the XCDs its workgroups fall to, each of which fetches its own copy
+// of the B rows, and 16 gathers of a row per XCD pay for that.  Narrow lanes
+// spread few workgroups over more CUs and each B row over fewer XCDs.  4-row
+// "orig", us at 4 / 2 / 1: 1211 x 9904 at 89 % x 199 164 / 132 / 109, 2699 x
+// 6439 at 98.5 % x 104 45 / 41 / 25, 4163 x 2281 at 92 % x 384 62 / 98 / 101,
+// 2424 x 524 at 71 % x 320 25 / 39 / 27.  Few rows of B under many columns are
+// bound by the stores of C: 63 x 199 at 58 % x 3168 5.9 / 7.5 / 8.0.  Over 350
+// drawn sizes (16..10000 rows, 16..12000 deep, 16..8192 columns, 50..99.7 %) it
+// takes 1.017 of the fastest width's time on average, the widest lane that
+// gives a workgroup per CU 1.038 and up to 1.67 times it.
+//   slices, wide: panels x 64- and x 256-column slices of the whole launch.
+static int default_lanes(int64_t slices, int64_t wide, int K, int64_t total_cols, int n) {
+    const int64_t cus = cu_count();
+    const int64_t per_xcd = std::min<int64_t>(8, (n + 255) / 256);  // eighths of the gathers that one XCD makes
+    if (n > 128 && (slices > 12 * cus || (total_cols * per_xcd >= 8 * 16 * (int64_t)K && 2 * wide >= cus) ||
+                    (K <= 256 && n >= 1024)))
+        return 4;
+    return n > 64 && slices > 10 * cus ? 2 : 1;
+}
+
 // Realise the GPU fields of a tile config for a matrix of K columns with
 // `total_cols` packed columns and B width n (the choices the reference's
 // heuristic JSON made per sparsity bucket are made here from the launch
 // geometry; the autotuner overrides them with measured choices).
-//
-// Lane width: the widest whose N tiles still give the chip a workgroup per CU
-// (a panel never spans two workgroups), since a wide lane gathers the same
-// bytes in fewer batches.  Both sides at 16 waves, 8-row "orig": 4096 x 1024
-// at 90 % x 200 runs 19.5 us at V = 4 (512 workgroups) and 31.6 at V = 1;
-// 1000 x 777 at 80 % x 200 runs 12.4 at V = 1 and 16.1 at V = 4 (125).  Two
-// floats pay only with half a round more.
 //
 // Waves: 8 at every size (plans of one group have to agree).  16 are about a
 // twentieth faster on small products and up to a half slower on large ones
@@ -615,12 +631,8 @@ static int cu_count() {
 // (0.72 to 1.08); with fewer tiles a panel's extra chunks only open a second
 // round (1.10 over 26).
 static void realise_config(srt_tile_config &c, int P, int M_r, int K, int K_tile, int64_t total_cols, int n) {
-    if (c.vec_width != 1 && c.vec_width != 2 && c.vec_width != 4) {
-        const int64_t cus = cu_count();
-        c.vec_width = n > 128 && 16 * (int64_t)P * ((n + 255) / 256) >= 15 * cus ? 4
-                      : n > 64 && 2 * (int64_t)P * ((n + 127) / 128) >= 3 * cus  ? 2
-                                                                                 : 1;
-    }
+    if (c.vec_width != 1 && c.vec_width != 2 && c.vec_width != 4)
+        c.vec_width = default_lanes((int64_t)P * ((n + 63) / 64), (int64_t)P * ((n + 255) / 256), K, total_cols, n);
     const bool own = c.waves_per_block < 1 || c.waves_per_block > kMaxWaves;
     if (own) c.waves_per_block = 8;
     if (c.nsplit < 1 || c.nsplit > c.waves_per_block) c.nsplit = c.waves_per_block;

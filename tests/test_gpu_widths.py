@@ -158,3 +158,14 @@ def test_lane_width_of_many_waves_stays_within_its_lds(srt):
     args = lambda V: (plan._h, B.data_ptr(), 512, C.data_ptr(), 512, 512, V, 0, ct.byref(out))
     assert fill(*args(2)) == 0
     assert fill(*args(4)) == srt._lib.SRT_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("M,K,s,N,V", [(1211, 9904, 0.887, 199, 1), (2699, 6439, 0.985, 104, 1), (4163, 2281, 0.92, 384, 4),
+                                       (2424, 524, 0.708, 320, 4), (63, 199, 0.583, 3168, 4), (512, 512, 0.95, 128, 1),
+                                       (16384, 256, 0.9, 128, 2)])
+def test_default_lane_width(srt, M, K, s, N, V):
+    """Sizes on either side of the lines of the default rule."""
+    import torch
+    csr = (torch.rand(M, K, device="cuda") >= s).float().to_sparse_csr()
+    plan = srt.MatMulSpecialized.from_csr(csr, N, mapping_id=srt.named_mapping(4, "orig"))
+    assert plan.get_config().vec_width == V
