@@ -100,7 +100,9 @@ typedef struct srt_tile_config {
                               chains run in column order): tiles of B rows staged in
                               LDS one after another, chunk_cols (1, 2, 4, 8) C rows
                               per wave, waves_per_block 4, 8 or 16, one chain per
-                              row (nsplit 1); 0 = choose (3 where it applies, else
+                              row (nsplit 1); 0 = choose (3 for an M_r = 1 mapping
+                              where its estimated time is the lower one and
+                              neither nsplit > 1 nor chunk_cols is given, else
                               global memory)                                      */
     int layout;            /* wave slots -> workgroups: 1 = panels in order, a panel
                               on kp waves as chunk_cols says; 2 = balanced: panels
@@ -222,6 +224,10 @@ int srt_plan_create_hybrid(int m, int k, int n, const float *Lx, const void *Lp,
 int srt_plan_dense_panels(const srt_plan *p, int *num_dense, int32_t *panel_rows, size_t *bytes);
 
 int srt_plan_get_config(const srt_plan *p, srt_tile_config *out);
+
+/* The streamed launch (b_staging 3, 16 waves) of least estimated time for an
+ * m x k matrix of nnz entries times n columns, and that time.  Host only. */
+int srt_stream_estimate(int m, int k, int64_t nnz, int n, int *vec_width, int *rows_per_wave, double *seconds);
 
 /* Bytes of packed A held on the device (MatMulSpecialized::require_storage). */
 int srt_plan_required_storage(const srt_plan *p, size_t *bytes);

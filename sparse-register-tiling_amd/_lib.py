@@ -104,6 +104,7 @@ SIGNATURES = {
     "srt_plan_schedule_bytes": (_i, [_vp, ct.POINTER(ct.c_size_t)]),
     "srt_plan_launch_shape": (_i, [_vp, _i, ct.POINTER(_i), ct.POINTER(_i)]),
     "srt_probe_launch_floor": (_i, [_i, _i, _i, _vp, _i64, _i, _vp, _vp]),
+    "srt_stream_estimate": (_i, [_i, _i, _i64, _i, ct.POINTER(_i), ct.POINTER(_i), ct.POINTER(ct.c_double)]),
     "srt_plan_split_counts": (_i, [_vp, _vp]),
     "srt_tile_split_counts": (_i, [_vp, _vp]),
     "srt_sort_and_encode_patterns": (_i, [_vp, _vp, _i, _vp, _vp, _vp]),

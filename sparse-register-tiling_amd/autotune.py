@@ -14,6 +14,7 @@ follows the heuristic file: bucket -> bcols -> ranked configs.
 """
 from __future__ import annotations
 
+import ctypes as ct
 import json
 import os
 import statistics
@@ -21,6 +22,7 @@ from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
+from . import _lib
 from .matmul import MatMulSpecialized, TileConfig
 from .mapping import named_mapping
 
@@ -439,33 +441,12 @@ def add_candidate(cache: "TuningCache", case, mapping: Tuple[int, str], shape: D
     return rec
 
 
-# Streamed execution (one row per panel, B tiles in LDS) against the gather
-# executor, for sizes the table does not hold.  Fitted to 90 sizes (M 512-4096,
-# K 512-4096, sparsity 0.70-0.95, N 128-2048; 256 CUs, 2.4 GHz).  Per lane
-# width V: clocks of a workgroup's B tile when staging bounds it, clocks per
-# entry, clocks per tile beside the entries.
-STREAM_COST = {1: (7000.0, 2.8, 4000.0), 2: (5600.0, 4.7, 2500.0), 4: (4800.0, 8.5, 2000.0)}
-STREAM_WAVES = 16
-
-
 def streamed_launch(M: int, K: int, nnz: int, N: int) -> Tuple[int, int, float]:
     """(lane width, rows per wave, estimated seconds) of the fastest streamed
-    launch.  A wide lane halves the LDS reads per product, a narrow one the
-    B bytes a workgroup stages; rows per wave fill the chip's 256 workgroups
-    once (a second round costs a whole pass).  A row's entries of a tile are
-    padded to four: 1.5 more on average."""
-    best = (1, 1, float("inf"))
-    for V, (staging, per_entry, per_tile) in STREAM_COST.items():
-        rows = 16 * STREAM_WAVES // V  # B rows of a tile
-        tiles = -(-max(K, 1) // rows)
-        for R in (1, 2, 4, 8):
-            groups = -(-M // (STREAM_WAVES * R)) * -(-max(N, 1) // (64 * V))
-            entries = STREAM_WAVES * R * (nnz / float(max(1, M * tiles)) + 1.5)
-            tile = max(staging, per_entry * entries + per_tile)
-            t = 2.2e-6 + -(-groups // 256) * tiles * tile / 2.4e9
-            if t < best[2]:
-                best = (V, R, t)
-    return best
+    launch (srt_stream_estimate, the rule of a streamed plan's own defaults)."""
+    V, R, seconds = ct.c_int(), ct.c_int(), ct.c_double()
+    _lib.call("srt_stream_estimate", M, K, nnz, N, ct.byref(V), ct.byref(R), ct.byref(seconds))
+    return V.value, R.value, seconds.value
 
 
 def gather_seconds(M: int, K: int, nnz: int, N: int) -> float:

@@ -671,22 +671,69 @@ static bool column_ordered(const ExecutorDesc *e) { return e->M_r == 1 && e->num
 
 static bool streamed(const srt_tile_config &c) { return c.b_staging == 3; }
 
+struct StreamChoice {
+    int V, R;
+    double seconds;
+};
+
+// The fastest streamed launch by a time model, over the lane widths V and rows
+// per wave R (a positive one is given) for W waves a workgroup.  A wide lane
+// halves the LDS reads per product, a narrow one the B bytes a workgroup stages;
+// rows per wave fill the chip's 16 waves a CU once (a second round costs a whole
+// pass).  A row's entries of a tile are padded to four: 1.5 more on average.
+// Per V: clocks of a CU's B tiles when staging bounds them, clocks per entry,
+// clocks per tile beside the entries.  Fitted to 90 sizes (M 512-4096, K
+// 512-4096, sparsity 0.70-0.95, N 128-2048; 256 CUs, 2.4 GHz).
+static StreamChoice stream_choice(int M, int K, int64_t nnz, int n, int V_given, int R_given, int W) {
+    static constexpr struct {
+        int V;
+        double staging, per_entry, per_tile;
+    } kCost[] = {{1, 7000.0, 2.8, 4000.0}, {2, 5600.0, 4.7, 2500.0}, {4, 4800.0, 8.5, 2000.0}};
+    StreamChoice best{1, 1, -1.0};
+    const int64_t at_once = 256 * 16 / W;
+    for (const auto &cost : kCost) {
+        if (V_given > 0 && cost.V != V_given) continue;
+        const int64_t rows = stream_tile_rows(cost.V, W), tiles = (std::max(K, 1) + rows - 1) / rows;
+        for (int R = 1; R <= 8; R *= 2) {
+            if (R_given > 0 && R != R_given) continue;
+            const int64_t groups = (int64_t)((M + (int64_t)W * R - 1) / ((int64_t)W * R)) *
+                                   ((std::max(n, 1) + 64 * cost.V - 1) / (64 * cost.V));
+            const double entries = 16.0 * R * ((double)nnz / (double)std::max<int64_t>(1, M * tiles) + 1.5);
+            const double tile = std::max(cost.staging, cost.per_entry * entries + cost.per_tile);
+            const double t = 2.2e-6 + (double)((groups + at_once - 1) / at_once) * tiles * tile / 2.4e9;
+            if (best.seconds < 0 || t < best.seconds) best = {cost.V, R, t};
+        }
+    }
+    return best;
+}
+
+// Whether a plan of one-row panels that leaves the executor open streams: its
+// estimate is a tenth below that of the gather executor (3.5 us, 1 ns per B row
+// and 0.2 us per 10^6 products; below 256 columns whole waves of 64), the bytes
+// of C on both sides.  Over 350 drawn sizes it takes 0.95 of the gather
+// executor's time on average and 1.07 at most.  Streaming walks all of B
+// whatever the nonzeros are: 38 x 7159 at 99.9 % x 365 takes 37 us and 4.9
+// gathered.  The rows beside a hybrid's dense panels also stream where a launch
+// is most of it (up to 5.5 us: at most 1.34 of the gather executor's time), one
+// chain per row like the panels beside them.
+static bool stream_pays(int M, int K, int64_t nnz, int n, bool hybrid) {
+    if (n < 32) return false;
+    const double stream = stream_choice(M, K, nnz, n, 0, 0, 16).seconds;
+    const double gather = 3.5e-6 + 1e-9 * K + 0.2e-12 * (double)nnz * (n >= 256 ? n : (n + 63) / 64 * 64);
+    const double store = 4.0 * M * (double)n / 2.5e12;
+    return stream + store < 0.9 * (gather + store) || (hybrid && stream < 5.5e-6);
+}
+
 // Realise the streamed launch of an M x K matrix at width n: lane width V,
-// waves per workgroup W, C rows per wave R (chunk_cols).
+// waves per workgroup W, C rows per wave R (chunk_cols), those not given by the
+// time model.
 static void realise_stream(srt_tile_config &c, int M, int K, int K_tile, int64_t nnz, int n) {
     if (c.waves_per_block != 4 && c.waves_per_block != 8 && c.waves_per_block != 16) c.waves_per_block = 16;
-    // One workgroup per CU in one round takes V * R = M n / (64 * waves of the
-    // chip); wide lanes read the LDS best, so V grows with the work first,
-    // then R (measured: 4 x 8 down to 2 x 2 lead at every size tried).
-    const int64_t vr = std::max<int64_t>(1, (int64_t)M * n / (64 * (int64_t)cu_count() * c.waves_per_block));
-    if (c.vec_width != 1 && c.vec_width != 2 && c.vec_width != 4)
-        c.vec_width = vr >= 16 && n > 128 ? 4 : vr >= 2 && n > 64 ? 2 : 1;
-    if (c.chunk_cols != 1 && c.chunk_cols != 2 && c.chunk_cols != 4 && c.chunk_cols != 8) {
-        const int64_t slices = (n + 64 * c.vec_width - 1) / (64 * c.vec_width);
-        const int64_t waves = (int64_t)cu_count() * c.waves_per_block;
-        const int64_t rows = ((int64_t)M * slices + waves - 1) / waves;
-        c.chunk_cols = rows <= 1 ? 1 : rows <= 2 ? 2 : rows <= 4 ? 4 : 8;
-    }
+    const int V = c.vec_width == 1 || c.vec_width == 2 || c.vec_width == 4 ? c.vec_width : 0;
+    const int R = pow2_upto8(c.chunk_cols) ? c.chunk_cols : 0;
+    const StreamChoice best = stream_choice(M, K, nnz, n, V, R, c.waves_per_block);
+    c.vec_width = best.V;
+    c.chunk_cols = best.R;
     if (c.xcd_remap != 0 && c.xcd_remap != 1) c.xcd_remap = 1;
     if (!pow2_upto8(c.unroll)) c.unroll = 4;
     if (c.layout != 1 && c.layout != 2) c.layout = 2;
@@ -1425,11 +1472,9 @@ static int mfma_ranges_for(srt_plan *p, int n) {
     return SRT_OK;
 }
 
-int srt_plan_create(int m, int k, int n, const float *Lx, const void *Lp, const void *Li,
-                    int index_bytes, const srt_tile_config *cfg, int nThreads,
-                    const char *executor_id, const srt_mapping *mapping, srt_stream_t stream,
-                    srt_plan **out) {
-    (void)nThreads;
+static int plan_create(int m, int k, int n, const float *Lx, const void *Lp, const void *Li, int index_bytes,
+                       const srt_tile_config *cfg, const char *executor_id, const srt_mapping *mapping,
+                       srt_stream_t stream, bool hybrid, srt_plan **out) {
     if (!out || !mapping) return fail(SRT_ERR_INVALID, "srt_plan_create: null argument");
     *out = nullptr;
     if (m < 0 || k < 0 || n < 0) return fail(SRT_ERR_INVALID, "negative dimension");
@@ -1458,8 +1503,12 @@ int srt_plan_create(int m, int k, int n, const float *Lx, const void *Lp, const 
     else srt_tile_config_default(&plan->cfg_user);
     plan->n_max = n;
     plan->cfg = plan->cfg_user;
-    if (column_ordered(exec) && (plan->cfg.b_staging == 0 || plan->cfg.b_staging == 3) && plan->cfg.matrix_cores != 1 &&
-        m > 0 && k > 0) {
+    // Open (b_staging 0): where it pays, unless the split of a panel's columns
+    // over waves is asked for, which only the gather executor has.
+    const srt_tile_config &u = plan->cfg_user;
+    const bool can = column_ordered(exec) && u.matrix_cores != 1 && m > 0 && k > 0;
+    const bool open = u.b_staging == 0 && u.nsplit <= 1 && u.chunk_cols < 1;
+    if (can && (u.b_staging == 3 || (open && stream_pays(m, k, plan->pk.total_cols, std::max(n, 1), hybrid)))) {
         realise_stream(plan->cfg, m, k, plan->pk.K_c, plan->pk.total_cols, std::max(n, 1));
         rc = build_stream(plan->pk, plan->cfg, plan->stream, (hipStream_t)stream);
         if (rc) {
@@ -1493,6 +1542,22 @@ int srt_plan_create(int m, int k, int n, const float *Lx, const void *Lp, const 
         return rc;
     }
     *out = plan.release();
+    return SRT_OK;
+}
+
+int srt_plan_create(int m, int k, int n, const float *Lx, const void *Lp, const void *Li, int index_bytes,
+                    const srt_tile_config *cfg, int nThreads, const char *executor_id, const srt_mapping *mapping,
+                    srt_stream_t stream, srt_plan **out) {
+    (void)nThreads;
+    return plan_create(m, k, n, Lx, Lp, Li, index_bytes, cfg, executor_id, mapping, stream, false, out);
+}
+
+int srt_stream_estimate(int m, int k, int64_t nnz, int n, int *vec_width, int *rows_per_wave, double *seconds) {
+    if (m < 0 || k < 0 || nnz < 0 || n < 0) return fail(SRT_ERR_INVALID, "negative dimension");
+    const StreamChoice c = stream_choice(m, k, nnz, n, 0, 0, 16);
+    if (vec_width) *vec_width = c.V;
+    if (rows_per_wave) *rows_per_wave = c.R;
+    if (seconds) *seconds = c.seconds;
     return SRT_OK;
 }
 
@@ -1591,7 +1656,7 @@ int srt_plan_create_hybrid(int m, int k, int n, const float *Lx, const void *Lp,
         SRT_HIP_TRY(hipMemcpyAsync(d_cv, cv2.data(), 4 * cv2.size(), hipMemcpyHostToDevice, s));
     }
     srt_plan *plan = nullptr;
-    SRT_TRY(srt_plan_create(m, k, n, d_cv, d_rp, d_ci, 8, cfg, 1, nullptr, mapping, stream, &plan));
+    SRT_TRY(plan_create(m, k, n, d_cv, d_rp, d_ci, 8, cfg, nullptr, mapping, stream, true, &plan));
     std::unique_ptr<srt_plan, void (*)(srt_plan *)> guard(plan, srt_plan_destroy);
     DensePart &dp = plan->dense;
     dp.ndense = nd;

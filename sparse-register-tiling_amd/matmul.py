@@ -42,7 +42,9 @@ class TileConfig:
     nsplit (waves sharing one panel; 1 keeps the reference's single chain),
     chunk_cols (target packed columns per wave), b_staging (1: B tile
     staged in LDS, 2: B rows read from global memory, 3: streamed, for
-    M_r = 1 mappings: tiles of B rows in LDS, chunk_cols rows per wave), layout (1: panels
+    M_r = 1 mappings: tiles of B rows in LDS, chunk_cols rows per wave; 0:
+    streamed where that is estimated to pay and neither nsplit > 1 nor
+    chunk_cols is given, else global memory), layout (1: panels
     laid into workgroups in order; 2: panels binned heaviest-first into
     whole rounds of the chip's CUs, slots given to the longest chunks) and
     matrix_cores (1: one v_mfma_f32_4x4x1_16b outer product per packed
