@@ -453,33 +453,40 @@ def gather_seconds(M: int, K: int, nnz: int, N: int) -> float:
     """Estimated seconds of the gather executor with the 4-row "orig" mapping
     on the same sizes: 4 us, 3 ns per B row (a panel's chain) and 0.2 us per
     10^6 products, times the packed columns per nonzero of a 4-row panel (one
-    B row gathered for each); below 256 columns whole waves of 64.  On 60
-    drawn sizes (M 256-4096, K 128-4096, N 1-4096, 66-97 % sparse) the lower
-    estimate takes 1.004 of the faster executor's time on average and 1.11 at
-    worst, on 60 others 1.013 and 1.53; without the chain and at 0.16 us it
-    took 1.03 and 1.60 on the first."""
+    B row gathered for each); below 256 columns whole waves of 64."""
     d = nnz / float(max(1, M * K))
     share = (1.0 - (1.0 - d) ** 4) / (4.0 * d) if d > 0 else 1.0
     width = N if N >= 256 else -(-N // 64) * 64
     return 4e-6 + 3e-9 * K + 0.2e-12 * share * nnz * width
 
 
+def stream_pays(M: int, K: int, nnz: int, N: int) -> bool:
+    """Whether the streamed executor's estimate is a tenth below the gather
+    executor's, the bytes of C at 2.5 TB/s on both sides.  Below 32 columns it
+    gains a tenth at best and loses a fifth where its tiles are short of rows
+    (3835 x 2508 at 70 % x 3: 54.9 us, 45.5 gathered).  Over 350 drawn sizes
+    (M 16-10000, K 16-12000, N 16-8192, 50-99.7 % sparse) two of the 49 it
+    streams are more than 5 % slower than the 4-row default of before (0.93);
+    without margin and stores 12 of 97 (0.87), and 1.013 of the faster
+    executor's time on average either way."""
+    _, _, seconds = streamed_launch(M, K, nnz, N)
+    store = 4.0 * M * N / 2.5e12
+    return N >= 32 and seconds + store < 0.9 * (gather_seconds(M, K, nnz, N) + store)
+
+
 def tuned_plan(csr: torch.Tensor, N: int, path: str = SHIPPED) -> MatMulSpecialized:
     """A plan with the best measured configuration of the tuning table for
     this shape, sparsity bucket and N (the reference's heuristic-JSON lookup,
     tools/paper/heuristic.py:26-50, experiment_runner.py:86-113).  Where the
-    table has no entry: streamed execution when its estimate is the lower
-    one, else the default configuration."""
+    table has no entry: streamed execution where that is estimated to pay,
+    else the default configuration."""
     M, K = csr.shape
     sparsity = 1.0 - csr.values().numel() / float(max(1, M * K))
     recs = TuningCache(path).get(M, K, sparsity, N)
     if not recs:
         nnz = csr.values().numel()
-        V, R, seconds = streamed_launch(M, K, nnz, N)
-        # Fewer than 32 columns: streaming gains a tenth at best, and loses a
-        # fifth where its tiles are short of rows (3835 x 2508 at 70 % x 3:
-        # 54.9 us, 45.5 gathered).
-        if N >= 32 and seconds < gather_seconds(M, K, nnz, N):
+        if stream_pays(M, K, nnz, N):
+            V, R, _ = streamed_launch(M, K, nnz, N)
             return MatMulSpecialized.from_csr(csr, N, mapping_id=named_mapping(1, "identity"),
                                               tile_config=TileConfig(b_staging=3, vec_width=V, waves_per_block=16,
                                                                      chunk_cols=R))

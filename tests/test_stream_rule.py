@@ -39,6 +39,15 @@ def test_estimate_is_the_model(srt):
         srt.autotune.streamed_launch(-1, 1, 1, 1)
 
 
+@pytest.mark.parametrize("M,K,s,N,streams", [
+    (4096, 1024, 0.8, 2048, True), (7669, 3554, 0.8781, 284, True), (12609, 214, 0.944, 309, True),
+    # slower streamed: 47 us (41 gathered), 24.0 (21.3), 6.4 (5.6), 6.2 (5.1)
+    (3150, 1957, 0.9663, 852, False), (1779, 138, 0.9534, 7704, False), (2725, 223, 0.9804, 299, False),
+    (503, 36, 0.9897, 5314, False), (3835, 2508, 0.7, 3, False), (512, 512, 0.95, 8, False)])
+def test_tuned_rule_streams_with_a_margin(srt, M, K, s, N, streams):
+    assert srt.autotune.stream_pays(M, K, int((1 - s) * M * K), N) == streams
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,K,s,N,cfg,streams", [
     (38, 7159, 0.9989, 365, {}, False),   # all of B for a few rows' entries: 37 us, 4.9 gathered
