@@ -1895,21 +1895,37 @@ struct srt_group {
 };
 
 // Problem table of a group for the given operands: each problem runs at its
-// own lane width (the widest of the plans' that its n fills and the LDS of its
-// reduction allows) and gets n_wblocks * ceil(n / 64 lanes) consecutive
-// workgroups; the launch is the widest problem's.
+// own lane width and gets n_wblocks * ceil(n / 64 lanes) consecutive
+// workgroups; the launch is the widest problem's.  A plan given a lane width
+// keeps it (narrower where its n or the LDS of its reduction does not fill it).
+// Left open, the plan's own width is for a launch alone on the chip; here the
+// rule counts the workgroups of all problems (the 16 layers of a network at 8
+// images, 8-row "orig": 254 us at the narrowest plan's own width, 146 so),
+// except for a problem whose own chains, about 1 us per four columns of a wave,
+// outlast the gathers of the whole group: few panels of a deep matrix in a small
+// group (44 x 1816 at 88 % x 784 beside five others: 23.1 us, 14.7 narrow).
 static int group_bind(srt_group &g, const float *const *B, const int64_t *ldb, float *const *C, const int64_t *ldc,
                       const int *n, hipStream_t s) {
     if (!B || !ldb || !C || !ldc || !n) return fail(SRT_ERR_INVALID, "srt_group: null operand array");
     const int cnt = (int)g.plans.size();
-    int most = 4;
-    for (int i = 0; i < cnt; ++i) most = std::min(most, g.plans[i]->cfg.vec_width);
+    int64_t slices = 0, wide = 0;
+    double gathers = 0.0;  // us
+    for (int i = 0; i < cnt; ++i) {
+        gathers += (double)g.plans[i]->pk.total_cols * std::max(n[i], 0) / 5e6;
+        slices += (int64_t)g.plans[i]->pk.P * ((std::max(n[i], 0) + 63) / 64);
+        wide += (int64_t)g.plans[i]->pk.P * ((std::max(n[i], 0) + 255) / 256);
+    }
     std::vector<int> lanes((size_t)cnt, 1);
     int V = 1, least = 4;
     for (int i = 0; i < cnt; ++i) {
         const srt_plan &p = *g.plans[i];
         if (n[i] < 0) return fail(SRT_ERR_INVALID, "srt_group: n must be >= 0");
-        int v = n[i] > 128 ? most : std::min(most, n[i] > 64 ? 2 : 1);
+        const int given = p.cfg_user.vec_width;
+        const int64_t own = (int64_t)p.pk.P * ((n[i] + 63) / 64), own4 = (int64_t)p.pk.P * ((n[i] + 255) / 256);
+        const bool alone = p.pk.P > 0 && (double)p.pk.total_cols / (4.0 * g.waves * p.pk.P) > gathers;
+        int v = given == 1 || given == 2 || given == 4
+                    ? std::min(p.cfg.vec_width, n[i] > 128 ? 4 : n[i] > 64 ? 2 : 1)
+                    : default_lanes(alone ? own : slices, alone ? own4 : wide, p.pk.K, p.pk.total_cols, n[i]);
         if (n[i] > 0 && p.pk.M > 0) {
             if (!B[i] || !C[i]) return fail(SRT_ERR_INVALID, "srt_group: null B or C");
             if (ldb[i] < n[i] || ldc[i] < n[i]) return fail(SRT_ERR_INVALID, "srt_group: ldb and ldc must be >= n");

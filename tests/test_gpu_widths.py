@@ -169,3 +169,40 @@ def test_default_lane_width(srt, M, K, s, N, V):
     csr = (torch.rand(M, K, device="cuda") >= s).float().to_sparse_csr()
     plan = srt.MatMulSpecialized.from_csr(csr, N, mapping_id=srt.named_mapping(4, "orig"))
     assert plan.get_config().vec_width == V
+
+
+def test_open_plans_of_a_group_take_the_group_s_lane_width(srt, oracle):
+    """Plans that leave the lane width open: a lone launch of these has too few
+    workgroups for wide lanes, the group has not.  One problem of few columns
+    does not narrow the others, a plan given a width keeps it; same bits."""
+    import torch
+    so, cb = oracle
+    mapping = srt.resolve_mapping(srt.named_mapping(4, "orig"))
+
+    def plan(A, N, **cfg):
+        rp, ci, v = srt.workloads.to_csr(A)
+        return srt.MatMulSpecialized(A.shape[0], A.shape[1], N, torch.from_numpy(v), torch.from_numpy(rp),
+                                     torch.from_numpy(ci), tile_config=srt.TileConfig(**cfg), mapping_id=mapping)
+
+    A = srt.workloads.magnitude_pruned(160, 300, 0.8, seed=1)
+    B = srt.workloads.dense_b(300, 400, seed=2)
+    assert plan(A, 400).get_config().vec_width == 1
+    for cfgs, narrow, want in (([{}] * 12, None, 4), ([{}] * 11 + [dict(vec_width=2)], None, 2), ([{}] * 12, 40, 1),
+                               ([{}] * 2, None, 1)):
+        plans = [plan(A, 400, **c) for c in cfgs]
+        n = [400] * len(plans)
+        if narrow:
+            n[3] = narrow
+        Bs = [torch.from_numpy(np.ascontiguousarray(B[:, :k])).cuda() for k in n]
+        Cs = [torch.full((160, k), float("nan"), device="cuda") for k in n]
+        g = srt.cnn.GroupedPlans(plans, Bs, Cs)
+        g()
+        torch.cuda.synchronize()
+        assert g.info()["vec_width"] == want
+        if narrow:  # 12 x 40 panels x 7 slices, 11 of them at four floats per lane: two workgroups a panel
+            assert g.info()["workgroups"] < 12 * 40 * 7
+        for p, C, k in zip(plans, Cs, n):
+            ref = cb.exec_packed(cb.pack_dense(A, 4, _oracle_table(so, 4, "orig")), np.ascontiguousarray(B[:, :k]),
+                                 nsplit=p.split_counts())
+            assert np.array_equal(C.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+        g.close()
