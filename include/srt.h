@@ -295,13 +295,14 @@ void srt_plan_destroy(srt_plan *p);
 
 /* ------------------------------------------------------------------------
  * Grouped execution: several plans (the 1x1-conv layers of a network, each
- * with its own B and C) as one kernel launch.  No counterpart in the
+ * with its own B and C) as one kernel launch (streamed plans, b_staging 3,
+ * each as one more on the same stream).  No counterpart in the
  * reference, whose benchmark runs one MatMulSpecialized per matrix
  * (cpp_testbed/src/spmm/nano/SpMM_SOP.h:178); every problem keeps the
  * per-plan semantics of srt_plan_execute, bit for bit.
  *
- * The plans must share one executor (mapping) and waves_per_block and live
- * on the current device.  Operands are bound at create / rebind (a device
+ * The plans, streamed ones aside, must share one executor (mapping) and
+ * waves_per_block; all live on the current device.  Operands are bound at create / rebind (a device
  * problem table is written and the stream synchronised); srt_group_execute
  * only launches, so it can be captured in a graph and replayed.
  * ---------------------------------------------------------------------- */
@@ -310,12 +311,13 @@ typedef struct srt_group srt_group;
 int srt_group_create(const srt_plan *const *plans, int count, const float *const *B, const int64_t *ldb,
                      float *const *C, const int64_t *ldc, const int *n, srt_stream_t stream, srt_group **out);
 /* Re-bind operands (same plans; shapes may change).  Not while a launch of
- * the group is pending or a graph holding it may replay. */
+ * the group is pending or a graph holding it may replay (capture it again: the
+ * operands of streamed plans are launch arguments). */
 int srt_group_rebind(srt_group *g, const float *const *B, const int64_t *ldb, float *const *C,
                      const int64_t *ldc, const int *n, srt_stream_t stream);
 int srt_group_execute(const srt_group *g, srt_stream_t stream);
 /* Lane width (floats per lane) of the group's narrowest problem (each runs at
- * its own), workgroups, LDS bytes. */
+ * its own), workgroups of all launches, LDS bytes of the grouped one. */
 int srt_group_info(const srt_group *g, int *vec_width, int *workgroups, int *lds_bytes);
 void srt_group_destroy(srt_group *g);
 

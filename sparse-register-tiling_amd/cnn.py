@@ -100,7 +100,8 @@ def activations(layers: Sequence[CnnLayer], batch: int, seed: int = 1, device="c
 class GroupedPlans:
     """Several MatMulSpecialized plans run as one grouped register-tiled
     launch: C_i = A_i . B_i for every i.  The plans must share a mapping
-    (executor) and waves_per_block."""
+    (executor) and waves_per_block; streamed plans may be among them, each a
+    launch of its own beside the grouped one."""
 
     def __init__(self, plans: Sequence[MatMulSpecialized], B: Sequence[torch.Tensor],
                  C: Sequence[torch.Tensor], n: Optional[Sequence[int]] = None,

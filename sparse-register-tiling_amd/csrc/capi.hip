@@ -819,8 +819,10 @@ static int run_executor(const Packed &pk, const Schedule &sch, const ExecutorDes
     return SRT_OK;
 }
 
-static int run_stream(const Packed &pk, const StreamSched &st, const srt_tile_config &cfg, const float *B, int64_t ldb,
-                      float *C, int64_t ldc, int n, hipStream_t s) {
+// Launch arguments of a streamed plan, checked (N = 0: nothing to launch).
+static int bind_stream(const Packed &pk, const StreamSched &st, const srt_tile_config &cfg, const float *B, int64_t ldb,
+                       float *C, int64_t ldc, int n, StreamLaunch &out) {
+    out = StreamLaunch{};
     if (n < 0) return fail(SRT_ERR_INVALID, "n must be >= 0");
     if (n == 0) return SRT_OK;
     if (!B || !C) return fail(SRT_ERR_INVALID, "null B or C");
@@ -828,8 +830,16 @@ static int run_stream(const Packed &pk, const StreamSched &st, const srt_tile_co
     // B rows are addressed with a 32-bit byte offset (buffer loads).
     if ((int64_t)pk.K * ldb * (int64_t)sizeof(float) > (int64_t)0xffffffffLL)
         return fail(SRT_ERR_UNSUPPORTED, "B larger than 4 GiB (K * ldb * 4 bytes)");
-    StreamLaunch a{st.blocks, st.first, st.rows_of, B, C, ldb, ldc, n, pk.K, st.V, st.R, st.waves, st.n_wg,
-                   cfg.xcd_remap};
+    out = StreamLaunch{st.blocks, st.first, st.rows_of, B, C, ldb, ldc, n, pk.K, st.V, st.R, st.waves, st.n_wg,
+                       cfg.xcd_remap};
+    return SRT_OK;
+}
+
+static int run_stream(const Packed &pk, const StreamSched &st, const srt_tile_config &cfg, const float *B, int64_t ldb,
+                      float *C, int64_t ldc, int n, hipStream_t s) {
+    StreamLaunch a;
+    const int rc = bind_stream(pk, st, cfg, B, ldb, C, ldc, n, a);
+    if (rc) return rc;
     SRT_HIP_TRY(launch_stream(a, s));
     return SRT_OK;
 }
@@ -1408,8 +1418,8 @@ static bool full_pattern(const ExecutorDesc *e) {
     return e && e->M_r == 4 && e->num_patterns == 1 && e->patterns[0] == 15;
 }
 
-// The gather schedule of a streamed plan (grouped and persistent launches run
-// it), built at the first need; other plans have it from their creation.
+// The gather schedule of a streamed plan (persistent launches run it), built at
+// the first need; other plans have it from their creation.
 static int ensure_gather(const srt_plan *cp) {
     if (!streamed(cp->cfg)) return SRT_OK;
     srt_plan *p = const_cast<srt_plan *>(cp);
@@ -1885,8 +1895,11 @@ void srt_plan_destroy(srt_plan *p) {
 // ------------------------------------------------------------ grouped plans
 }  // extern "C"
 
+// The gather plans run as one launch over a device table; a streamed plan among
+// them (its entries are of another kind, and it is faster by itself) as its own.
 struct srt_group {
     std::vector<const srt_plan *> plans;
+    std::vector<StreamLaunch> streams;
     const ExecutorDesc *exec = nullptr;
     int waves = 0, V = 1, least = 1, total_blocks = 0, xcd_remap = 1, device = 0;
     size_t lds = 0;
@@ -1911,15 +1924,24 @@ static int group_bind(srt_group &g, const float *const *B, const int64_t *ldb, f
     int64_t slices = 0, wide = 0;
     double gathers = 0.0;  // us
     for (int i = 0; i < cnt; ++i) {
+        if (streamed(g.plans[i]->cfg)) continue;
         gathers += (double)g.plans[i]->pk.total_cols * std::max(n[i], 0) / 5e6;
         slices += (int64_t)g.plans[i]->pk.P * ((std::max(n[i], 0) + 63) / 64);
         wide += (int64_t)g.plans[i]->pk.P * ((std::max(n[i], 0) + 255) / 256);
     }
     std::vector<int> lanes((size_t)cnt, 1);
+    std::vector<StreamLaunch> streams;
     int V = 1, least = 4;
     for (int i = 0; i < cnt; ++i) {
         const srt_plan &p = *g.plans[i];
         if (n[i] < 0) return fail(SRT_ERR_INVALID, "srt_group: n must be >= 0");
+        if (streamed(p.cfg)) {
+            StreamLaunch a;
+            SRT_TRY(bind_stream(p.pk, p.stream, p.cfg, B[i], ldb[i], C[i], ldc[i], n[i], a));
+            if (a.N > 0) streams.push_back(a);
+            least = std::min(least, p.stream.V);
+            continue;
+        }
         const int given = p.cfg_user.vec_width;
         const int64_t own = (int64_t)p.pk.P * ((n[i] + 63) / 64), own4 = (int64_t)p.pk.P * ((n[i] + 255) / 256);
         const bool alone = p.pk.P > 0 && (double)p.pk.total_cols / (4.0 * g.waves * p.pk.P) > gathers;
@@ -1954,7 +1976,7 @@ static int group_bind(srt_group &g, const float *const *B, const int64_t *ldb, f
     size_t lds = 0;
     for (int i : order) {
         const srt_plan &p = *g.plans[i];
-        if (n[i] == 0 || p.pk.M == 0 || p.sch.n_wblocks == 0) continue;
+        if (n[i] == 0 || p.pk.M == 0 || p.sch.n_wblocks == 0 || streamed(p.cfg)) continue;
         ExecProblem q{};
         q.prog = p.sch.prog;
         q.desc = p.sch.desc;
@@ -1988,6 +2010,7 @@ static int group_bind(srt_group &g, const float *const *B, const int64_t *ldb, f
         SRT_HIP_TRY(hipStreamSynchronize(s));
     }
     g.h_probs = std::move(t);
+    g.streams = std::move(streams);
     g.V = V;
     g.least = least;
     g.total_blocks = (int)total;
@@ -2008,10 +2031,11 @@ int srt_group_create(const srt_plan *const *plans, int count, const float *const
     SRT_HIP_TRY(hipGetDevice(&g->device));
     for (int i = 0; i < count; ++i) {
         const srt_plan *p = plans[i];
-        SRT_TRY(ensure_gather(p));
         if (p->device != g->device) return fail(SRT_ERR_INVALID, "srt_group_create: plan belongs to another device");
         if (p->dense.ndense) return fail(SRT_ERR_UNSUPPORTED, "srt_group_create: hybrid plans execute alone");
-        if (i == 0) {
+        g->plans.push_back(p);
+        if (streamed(p->cfg)) continue;
+        if (!g->exec) {
             g->exec = p->exec;
             g->waves = p->sch.waves_per_block;
             g->xcd_remap = p->cfg.xcd_remap;
@@ -2022,9 +2046,9 @@ int srt_group_create(const srt_plan *const *plans, int count, const float *const
         }
         if (p->sch.unroll != 4)
             return fail(SRT_ERR_UNSUPPORTED, "srt_group_create: grouped launches need unroll 4");
-        g->plans.push_back(p);
     }
-    if (!g->exec->grouped[0]) return fail(SRT_ERR_UNSUPPORTED, "srt_group_create: executor has no grouped variant");
+    if (g->exec && !g->exec->grouped[0])
+        return fail(SRT_ERR_UNSUPPORTED, "srt_group_create: executor has no grouped variant");
     int rc = group_bind(*g, B, ldb, C, ldc, n, (hipStream_t)stream);
     if (rc) {
         hipFree(g->d_probs);
@@ -2045,11 +2069,13 @@ int srt_group_execute(const srt_group *g, srt_stream_t stream) {
     int dev = -1;
     SRT_HIP_TRY(hipGetDevice(&dev));
     if (dev != g->device) return fail(SRT_ERR_INVALID, "group belongs to another device");
-    if (g->total_blocks == 0) return SRT_OK;
-    ExecGroupedFn fn = g->exec->grouped[log2_small(g->V)];
-    if (!fn) return fail(SRT_ERR_UNSUPPORTED, "grouped executor variant not generated");
-    SRT_HIP_TRY(fn(g->d_probs, (int)g->h_probs.size(), g->total_blocks, g->waves, g->lds, g->xcd_remap,
-                   (hipStream_t)stream));
+    if (g->total_blocks > 0) {
+        ExecGroupedFn fn = g->exec->grouped[log2_small(g->V)];
+        if (!fn) return fail(SRT_ERR_UNSUPPORTED, "grouped executor variant not generated");
+        SRT_HIP_TRY(fn(g->d_probs, (int)g->h_probs.size(), g->total_blocks, g->waves, g->lds, g->xcd_remap,
+                       (hipStream_t)stream));
+    }
+    for (const StreamLaunch &a : g->streams) SRT_HIP_TRY(launch_stream(a, (hipStream_t)stream));
     return SRT_OK;
 }
 
@@ -2127,7 +2153,11 @@ int srt_exec_persistent_execute(const srt_plan *proto, int vec_width, const srt_
 int srt_group_info(const srt_group *g, int *vec_width, int *workgroups, int *lds_bytes) {
     if (!g) return fail(SRT_ERR_INVALID, "null group");
     if (vec_width) *vec_width = g->least;
-    if (workgroups) *workgroups = g->total_blocks;
+    if (workgroups) {
+        int64_t all = g->total_blocks;
+        for (const StreamLaunch &a : g->streams) all += (int64_t)a.n_wg * ((a.N + 64 * a.V - 1) / (64 * a.V));
+        *workgroups = (int)std::min<int64_t>(all, 0x7fffffff);
+    }
     if (lds_bytes) *lds_bytes = (int)g->lds;
     return SRT_OK;
 }

@@ -151,3 +151,60 @@ def test_alternating_widths_reuse_their_schedules(srt, oracle):
             free = torch.cuda.mem_get_info()[0]
     assert len(shapes) == 2
     assert torch.cuda.mem_get_info()[0] >= free  # a further copy of the entries is 5 MB
+
+
+def test_tuned_plans_group(srt, oracle):
+    """Tuned plans of sizes the table does not hold, some streamed, some not, in
+    one group: the bits of their own launches, captured and re-bound."""
+    import torch
+    sizes = [(300, 220, 0.9, 100), (4096, 1024, 0.8, 640), (129, 500, 0.8, 33), (4096, 500, 0.75, 1000), (64, 64, 0.9, 5)]
+    plans, Bs, Cs, refs = [], [], [], []
+    for i, (M, K, s, N) in enumerate(sizes):
+        g = torch.Generator(device="cuda").manual_seed(i)
+        A = torch.randn((M, K), generator=g, device="cuda") * (torch.rand((M, K), generator=g, device="cuda") >= s)
+        p = srt.autotune.tuned_plan(A.to_sparse_csr(), N)
+        B = torch.rand((K, N + 3), generator=g, device="cuda")[:, 1:1 + N]
+        C = torch.full((M, N), float("nan"), device="cuda")
+        ref = torch.empty_like(C)
+        p(ref, B)
+        plans.append(p), Bs.append(B), Cs.append(C), refs.append(ref)
+    streamed = [p.get_config().b_staging == 3 for p in plans]
+    assert any(streamed) and not all(streamed)
+    g = srt.cnn.GroupedPlans(plans, Bs, Cs)
+    g()
+    torch.cuda.synchronize()
+    for C, ref in zip(Cs, refs):
+        assert torch.equal(C, ref)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        g()
+    for _ in range(3):
+        for C in Cs:
+            C.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for C, ref in zip(Cs, refs):
+            assert torch.equal(C, ref)
+    del graph
+    n = [max(1, s[3] // 3) for s in sizes]
+    n[1], n[4] = 0, 0  # nothing to do for a streamed one and another
+    part = [torch.full((s[0], max(k, 1)), 7.0, device="cuda") for s, k in zip(sizes, n)]
+    g.rebind(Bs, part, n=n)
+    g()
+    torch.cuda.synchronize()
+    for C, ref, k in zip(part, refs, n):
+        assert torch.equal(C[:, :k], ref[:, :k]) and (k or bool((C == 7.0).all()))
+    g.close()
+    only = srt.cnn.GroupedPlans([p for p, s in zip(plans, streamed) if s], [b for b, s in zip(Bs, streamed) if s],
+                                [c for c, s in zip(Cs, streamed) if s])
+    for C in Cs:
+        C.zero_()
+    only()
+    torch.cuda.synchronize()
+    for C, ref, s in zip(Cs, refs, streamed):
+        assert torch.equal(C, ref) if s else not bool(C.any())
+    assert only.info()["workgroups"] > 0
+    # what cannot share a launch is still refused beside a streamed plan
+    other = srt.MatMulSpecialized.from_csr(torch.eye(64).to_sparse_csr(), 5, mapping_id=srt.named_mapping(8, "orig"))
+    with pytest.raises(srt.SrtError, match="executors"):
+        srt.cnn.GroupedPlans([plans[1], plans[4], other], [Bs[1], Bs[4], Bs[4]], [Cs[1], Cs[4], Cs[4]])
