@@ -24,7 +24,7 @@ import torch
 
 from . import _lib
 from .matmul import MatMulSpecialized, TileConfig
-from .mapping import named_mapping
+from .mapping import Mapping, named_mapping
 
 DEFAULT_MAPPINGS = [(8, "orig"), (8, "identity"), (4, "identity"), (4, "orig")]
 # GPU realisations tried per mapping: B path x lane width x unroll x (waves, split).
@@ -474,25 +474,45 @@ def stream_pays(M: int, K: int, nnz: int, N: int) -> bool:
     return N >= 32 and seconds + store < 0.9 * (gather_seconds(M, K, nnz, N) + store)
 
 
+def plan_choice(csr: torch.Tensor, N: int, path: str = SHIPPED) -> Tuple[Mapping, Optional[TileConfig]]:
+    """(mapping, configuration or None for the default one) of tuned_plan."""
+    M, K = csr.shape
+    nnz = csr.values().numel()
+    recs = TuningCache(path).get(M, K, 1.0 - nnz / float(max(1, M * K)), N)
+    if recs:
+        (M_r, name), cfg = best_config(recs)
+        return named_mapping(M_r, name), cfg
+    if stream_pays(M, K, nnz, N):
+        V, R, _ = streamed_launch(M, K, nnz, N)
+        return named_mapping(1, "identity"), TileConfig(b_staging=3, vec_width=V, waves_per_block=16, chunk_cols=R)
+    return named_mapping(4, "orig"), None
+
+
 def tuned_plan(csr: torch.Tensor, N: int, path: str = SHIPPED) -> MatMulSpecialized:
     """A plan with the best measured configuration of the tuning table for
     this shape, sparsity bucket and N (the reference's heuristic-JSON lookup,
     tools/paper/heuristic.py:26-50, experiment_runner.py:86-113).  Where the
     table has no entry: streamed execution where that is estimated to pay,
     else the default configuration."""
-    M, K = csr.shape
-    sparsity = 1.0 - csr.values().numel() / float(max(1, M * K))
-    recs = TuningCache(path).get(M, K, sparsity, N)
-    if not recs:
-        nnz = csr.values().numel()
-        if stream_pays(M, K, nnz, N):
-            V, R, _ = streamed_launch(M, K, nnz, N)
-            return MatMulSpecialized.from_csr(csr, N, mapping_id=named_mapping(1, "identity"),
-                                              tile_config=TileConfig(b_staging=3, vec_width=V, waves_per_block=16,
-                                                                     chunk_cols=R))
-        return MatMulSpecialized.from_csr(csr, N, mapping_id=named_mapping(4, "orig"))
-    (M_r, name), cfg = best_config(recs)
-    return MatMulSpecialized.from_csr(csr, N, mapping_id=named_mapping(M_r, name), tile_config=cfg)
+    mapping, cfg = plan_choice(csr, N, path)
+    return MatMulSpecialized.from_csr(csr, N, mapping_id=mapping, tile_config=cfg)
+
+
+def hybrid_choices(csr: torch.Tensor, N: int, plan: MatMulSpecialized, path: str = SHIPPED
+                   ) -> Tuple[Mapping, List[Optional[TileConfig]]]:
+    """(mapping, configurations to time) of the register-tiled rows of a tuned
+    hybrid beside `plan`, the tuned plan of the whole matrix: its mapping, with
+    what its configuration leaves open chosen for the panels that are left, and
+    as the whole matrix has it.  Neither leads: 1956 x 1351 at 69 % x 177, 70 of
+    123 panels dense, takes 43.7 us with the first and 33.7 with the second, 792
+    x 1275 at 68 % x 249, 2 of 50, 23.5 and 30.0.  Where the plan streams, the
+    default alone, since the few rows a hybrid leaves would stream all of B
+    (4096 x 1024 x 512: 71.9 us with 3 of 256 panels left to streaming, 55.9
+    with 7 left to the gather)."""
+    mapping, cfg = plan_choice(csr, N, path)
+    if cfg is not None and cfg.b_staging == 3:
+        return named_mapping(4, "orig"), [None]
+    return mapping, [cfg, plan.get_config()]
 
 
 HYBRID_THRESHOLDS = (0.2, 0.25, 0.3, 0.35, 0.4)
@@ -501,10 +521,10 @@ HYBRID_THRESHOLDS = (0.2, 0.25, 0.3, 0.35, 0.4)
 def tuned_hybrid(csr: torch.Tensor, N: int, thresholds: Sequence[float] = HYBRID_THRESHOLDS, reps: int = 30,
                  path: str = SHIPPED) -> Tuple[MatMulSpecialized, Dict[str, object]]:
     """The fastest of the tuned plain plan and its hybrids (16-row panels at
-    least `threshold` dense on FP32 matrix cores, the rest register-tiled
-    with the plain plan's mapping and configuration, the default one where
-    that streams), graph-timed on the device at width N.  The reference fixes its dense-tile threshold at 0.30
-    (sbench/padding_reordering.py:36); here each threshold that yields a
+    least `threshold` dense on FP32 matrix cores, the rest register-tiled as
+    hybrid_choices says), graph-timed on the device at width N.  The reference
+    fixes its dense-tile threshold at 0.30 (sbench/padding_reordering.py:36);
+    here each threshold that yields a
     different set of dense panels is timed and the measurement decides.
     Returns the plan and a report {"plain_s", "choice": threshold or None,
     "candidates": [(threshold, dense panels, seconds)]}; the other plans are
@@ -517,27 +537,28 @@ def tuned_hybrid(csr: torch.Tensor, N: int, thresholds: Sequence[float] = HYBRID
     best = tuned_plan(csr, N, path)
     best_s = time_graph(lambda: best(C, B), reps=reps)
     report: Dict[str, object] = {"plain_s": best_s, "choice": None, "candidates": []}
-    cfg, mapping = best.get_config(), best.mapping
-    if cfg.b_staging == 3:
-        # the few rows a hybrid leaves would stream all of B: the gather
-        # default instead (4096 x 1024 x 512: 71.9 us with 3 of 256 panels
-        # left to streaming, 55.9 with 7 left to the gather)
-        cfg, mapping = None, named_mapping(4, "orig")
+    mapping, configs = hybrid_choices(csr, N, best, path)
     seen = set()
     for tau in sorted(thresholds):
-        hp = MatMulSpecialized.from_csr(csr, N, mapping_id=mapping, tile_config=cfg, dense_threshold=tau)
-        rows = tuple(hp.dense_panels()["rows"])
-        if not rows or rows in seen:  # no dense panel (the plain plan) or a set already timed
-            hp.close()
-            continue
-        seen.add(rows)
-        t = time_graph(lambda: hp(C, B), reps=reps)
-        report["candidates"].append((tau, len(rows), t))
-        if t < best_s:
-            best.close()
-            best, best_s, report["choice"] = hp, t, tau
-        else:
-            hp.close()
+        rows, fastest, launches = None, None, []
+        for cfg in configs:
+            hp = MatMulSpecialized.from_csr(csr, N, mapping_id=mapping, tile_config=cfg, dense_threshold=tau)
+            rows = tuple(hp.dense_panels()["rows"])
+            # no dense panel (the plain plan), a set or a launch already timed
+            if not rows or rows in seen or hp.get_config() in launches:
+                hp.close()
+                continue
+            launches.append(hp.get_config())
+            t = time_graph(lambda: hp(C, B), reps=reps)
+            fastest = t if fastest is None else min(fastest, t)
+            if t < best_s:
+                best.close()
+                best, best_s, report["choice"] = hp, t, tau
+            else:
+                hp.close()
+        if fastest is not None:
+            seen.add(rows)
+            report["candidates"].append((tau, len(rows), fastest))
     return best, report
 
 

@@ -163,3 +163,45 @@ def test_tuned_hybrid_chooses_by_measurement(srt, oracle):
     plan2, rep2 = at.tuned_hybrid(torch.from_numpy(A2).to_sparse_csr(), 256)
     assert rep2["choice"] is None and rep2["candidates"] == [] and plan2.dense_panels()["count"] == 0
     plan2.close()
+
+
+def test_tuned_hybrids_also_try_the_launch_for_the_panels_that_are_left(srt, monkeypatch):
+    """Off the table the rows beside the dense panels are timed at the lane
+    width and chunk of the default rule for those rows and at those of all rows;
+    the faster is reported, and taken if it beats the plain plan."""
+    import torch
+    at = srt.autotune
+    M, K, N = 2048, 600, 300
+    g = torch.Generator().manual_seed(2)
+    density = torch.full((M, 1), 0.5)
+    density[-256:] = 0.05  # 16 of 128 panels stay register-tiled
+    A = (torch.rand((M, K), generator=g) < density).float().to_sparse_csr()
+    real, timed = at.time_graph, []
+
+    def time_graph(launch, reps=50):
+        timed.append(real(launch, reps=reps))
+        return timed[-1]
+
+    monkeypatch.setattr(at, "time_graph", time_graph)
+    made, build = [], srt.MatMulSpecialized.from_csr.__func__
+
+    def from_csr(cls, *a, **kw):
+        made.append((kw, build(cls, *a, **kw)))
+        return made[-1][1]
+
+    monkeypatch.setattr(srt.MatMulSpecialized, "from_csr", classmethod(from_csr))
+    plan, rep = at.tuned_hybrid(A, N, thresholds=(0.3,), reps=3)
+    if made[0][1] is not plan:
+        assert rep["choice"] == 0.3
+    assert len(timed) == 3 and rep["candidates"] == [(0.3, 112, min(timed[1:]))]
+    assert made[1][0]["tile_config"] is None and made[2][0]["tile_config"] is not None
+    rest = A.to_dense()[-256:].to_sparse_csr()
+    alone = build(srt.MatMulSpecialized, rest, N, mapping_id=made[1][0]["mapping_id"]).get_config()
+    hybrid = build(srt.MatMulSpecialized, A, N, **made[1][0]).get_config()
+    assert (hybrid.vec_width, hybrid.chunk_cols) == (alone.vec_width, alone.chunk_cols)
+    assert made[2][0]["tile_config"].vec_width != hybrid.vec_width
+    B = torch.rand((K, N), device="cuda")
+    C = torch.empty((M, N), device="cuda")
+    plan(C, B)
+    Ad = A.to_dense().cuda().double()
+    assert bool(((C.double() - Ad @ B.double()).abs() <= (Ad @ B.double()) * (K + 40) * 2.0 ** -24).all())
