@@ -352,8 +352,9 @@ struct DensePart {
     size_t ws_bytes = 0;
     std::vector<void *> retired_ws;
     int reserve(int n) {
-        const size_t need = dense_panels_workspace_bytes(ndense, G, n);
+        size_t need = dense_panels_workspace_bytes(ndense, G, n);
         if (need <= ws_bytes) return SRT_OK;
+        need = std::max(need, 2 * ws_bytes);  // all that are kept hold less than the last
         void *w = nullptr;
         const hipError_t e = hipMalloc(&w, need);
         if (e != hipSuccess) return fail(SRT_ERR_NOMEM, std::string("hipMalloc failed: ") + hipGetErrorString(e));

@@ -373,14 +373,20 @@ DenseGrid dense_grid(int ndense, int G, int N, size_t ws_words) {
 
 }  // namespace
 
-// What 128 x 128 tiles with a workgroup per range would take; groups are fewer
-// and the padding of smaller tiles is less, so no launch takes more.
+// What 128 x 128 tiles with a workgroup per range would take at n columns or
+// any fewer (fewer columns are split further, so they may take more), at most
+// 256 tiles or 16 MB; groups are fewer and the padding of smaller tiles is
+// less, so no launch takes more.
 size_t dense_panels_workspace_bytes(int ndense, int G, int n) {
     if (ndense <= 0 || n <= 0) return 0;
-    int each = 0;
-    const int ranges = dense_ranges(ndense, std::max(1, (G + kSG - 1) / kSG), n, &each);
-    if (ranges <= 1) return 0;
-    return (size_t)ranges * ((ndense + 7) / 8) * ((n + 127) / 128) * tile_words(8, 8) * sizeof(f32x4);
+    const int stages = std::max(1, (G + kSG - 1) / kSG), pt = (ndense + 7) / 8;
+    int64_t most = 0;
+    for (int nt = 1; nt <= (n + 127) / 128 && (int64_t)pt * nt <= 128; ++nt) {
+        int each = 0;
+        const int ranges = dense_ranges(ndense, stages, 128 * nt, &each);
+        if (ranges > 1) most = std::max(most, (int64_t)ranges * pt * nt);
+    }
+    return (size_t)most * tile_words(8, 8) * sizeof(f32x4);
 }
 
 template <int kTP, int kNTiles>

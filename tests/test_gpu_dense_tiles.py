@@ -45,3 +45,26 @@ def test_tiles_and_splits(srt, mkn):
     part = torch.full((M, n), float("nan"), device="cuda")
     plan(part, B[:, :n].contiguous())
     assert bool(((part.double() - Ad @ B[:, :n].double()).abs() <= bound[:, :n] + 1e-30).all())
+
+
+@pytest.mark.parametrize("M,K,widths", [(1024, 4096, (1600, 900, 512, 300, 100, 1)), (512, 2000, (4096, 700, 256)),
+                                        (100, 300, (5000, 129))])
+def test_narrower_products_split_as_in_a_plan_of_their_own(srt, M, K, widths):
+    """Fewer columns than a plan was made for: the bits of a plan made for them."""
+    import torch
+    g = torch.Generator().manual_seed(M + K)
+    A = (torch.randn(M, K, generator=g) * (torch.rand(M, K, generator=g) < 0.5)).to_sparse_csr().cuda()
+
+    def make(n):
+        return srt.MatMulSpecialized.from_csr(A, n, mapping_id=srt.named_mapping(4, "orig"), dense_threshold=0.2)
+
+    wide = make(widths[0])
+    for n in widths:
+        print("narrow", M, K, widths[0], n, flush=True)
+        B = torch.randn((K, n), generator=g).cuda()
+        out, own = (torch.full((M, n), float("nan"), device="cuda") for _ in range(2))
+        plan = make(n)
+        wide(out, B)
+        plan(own, B)
+        torch.cuda.synchronize()
+        assert torch.equal(out, own)
