@@ -23,10 +23,11 @@
 // without, 264 with).  Per stage: the next stage's global loads are issued
 // first, the MFMAs of group q run while group q + 1's operands are read from
 // LDS, the next stage's words are written to the other buffer in the middle of
-// group 2, and the one barrier sits before group 3, whose MFMAs hide the next
-// stage's first reads.  Loads two stages ahead gave no more (156 us against
-// 154 at 1024 x 16384 x 512): large products run at 0.76 of the matrix cores'
-// cycles.
+// group 1 (in group 2 they hold up the narrow B loads of widths that 4 does not
+// divide: 720 x 2751 x 727 takes 49.0 us, 44.8 so), and the one barrier sits
+// before group 3, whose MFMAs hide the next stage's first reads.  Loads two
+// stages ahead gave no more (156 us against 154 at 1024 x 16384 x 512): large
+// products run at 0.76 of the matrix cores' cycles.
 //
 // K is cut into ranges, one chain of additions each, and ranges into at most
 // eight groups; a range's sum joins its group's, the groups' sums are added in
@@ -192,9 +193,9 @@ __global__ void __launch_bounds__(kThreads)
             mm(0);
             rd(buf, 2, 0);
             mm(1);
-            rd(buf, 3, 1);
             write_a(buf ^ 1);
             write_b(buf ^ 1);
+            rd(buf, 3, 1);
             mm(0);
             // that order, interleaved: global loads first; each group's next
             // operands after its first two MFMAs; the other buffer's writes in
@@ -205,12 +206,12 @@ __global__ void __launch_bounds__(kThreads)
             __builtin_amdgcn_sched_group_barrier(0x008, kMF - kH, 0);
             __builtin_amdgcn_sched_group_barrier(0x008, kH, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, kRD, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, kMF - kH, 0);
-            __builtin_amdgcn_sched_group_barrier(0x008, kH, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, kRD, 0);
             __builtin_amdgcn_sched_group_barrier(0x008, kMF / 2 - kH, 0);
             __builtin_amdgcn_sched_group_barrier(0x200, kAW + kBC, 0);
             __builtin_amdgcn_sched_group_barrier(0x008, kMF / 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, kH, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, kRD, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, kMF - kH, 0);
             __builtin_amdgcn_sched_barrier(0);
             __syncthreads();
             __builtin_amdgcn_sched_barrier(0);
