@@ -1426,6 +1426,9 @@ static int ensure_gather(const srt_plan *cp) {
     srt_plan *p = const_cast<srt_plan *>(cp);
     std::lock_guard<std::mutex> g(p->mu);
     if (p->sch.desc) return SRT_OK;
+    int dev = -1;  // it is built in the current device's memory
+    SRT_HIP_TRY(hipGetDevice(&dev));
+    if (dev != p->device) return fail(SRT_ERR_INVALID, "plan belongs to another device");
     srt_tile_config c = p->cfg_user;
     c.b_staging = 2;
     c.chunk_cols = 0;

@@ -208,3 +208,20 @@ def test_tuned_plans_group(srt, oracle):
     other = srt.MatMulSpecialized.from_csr(torch.eye(64).to_sparse_csr(), 5, mapping_id=srt.named_mapping(8, "orig"))
     with pytest.raises(srt.SrtError, match="executors"):
         srt.cnn.GroupedPlans([plans[1], plans[4], other], [Bs[1], Bs[4], Bs[4]], [Cs[1], Cs[4], Cs[4]])
+
+
+def test_gather_schedule_is_built_on_the_plan_s_device_only(srt):
+    """A problem table entry of a streamed plan, asked for with another GPU
+    current: refused, and built when its own is."""
+    import ctypes as ct
+
+    import torch
+    if torch.cuda.device_count() < 2:
+        pytest.skip("needs two GPUs")
+    A = srt.workloads.magnitude_pruned(64, 100, 0.7, seed=3)
+    plan = _plan(srt, torch, A, 64)
+    out = (ct.c_uint8 * 128)()
+    fill = srt._lib.lib().srt_exec_problem_fill
+    with torch.cuda.device(1):
+        assert fill(plan._h, None, 64, None, 64, 0, 1, 0, ct.byref(out)) == srt._lib.SRT_ERR_INVALID
+    assert fill(plan._h, None, 64, None, 64, 0, 1, 0, ct.byref(out)) == 0
