@@ -632,6 +632,7 @@ static int default_lanes(int64_t slices, int64_t wide, int K, int64_t total_cols
 // (0.72 to 1.08); with fewer tiles a panel's extra chunks only open a second
 // round (1.10 over 26).
 static void realise_config(srt_tile_config &c, int P, int M_r, int K, int K_tile, int64_t total_cols, int n) {
+    if (c.b_staging == 3) c.chunk_cols = c.nsplit = 0;  // a streamed plan's, C rows per wave: nothing of this executor
     if (c.vec_width != 1 && c.vec_width != 2 && c.vec_width != 4)
         c.vec_width = default_lanes((int64_t)P * ((n + 63) / 64), (int64_t)P * ((n + 255) / 256), K, total_cols, n);
     const bool own = c.waves_per_block < 1 || c.waves_per_block > kMaxWaves;

@@ -71,3 +71,17 @@ def test_open_plans_stream_where_it_pays(srt, M, K, s, N, cfg, streams):
         assert (real.vec_width, real.chunk_cols, real.waves_per_block) == (V, R, 16)
     if cfg.get("nsplit", 0) > 1 or cfg.get("chunk_cols"):
         assert (real.nsplit, real.chunk_cols) == (cfg.get("nsplit", real.nsplit), cfg.get("chunk_cols", real.chunk_cols))
+
+
+@pytest.mark.gpu
+def test_a_streamed_configuration_on_another_mapping(srt):
+    """Its rows per wave are not taken for packed columns per wave."""
+    import torch
+    csr = (torch.rand(2048, 1024, device="cuda") >= 0.8).float().to_sparse_csr()
+    cfg = srt.MatMulSpecialized.from_csr(csr, 512, mapping_id=srt.named_mapping(1, "identity"),
+                                         tile_config=srt.TileConfig(b_staging=3)).get_config()
+    assert cfg.b_staging == 3 and cfg.chunk_cols <= 8 and cfg.nsplit == 1
+    real = srt.MatMulSpecialized.from_csr(csr, 512, mapping_id=srt.named_mapping(4, "orig"), tile_config=cfg).get_config()
+    same = srt.TileConfig(vec_width=cfg.vec_width, waves_per_block=cfg.waves_per_block)
+    want = srt.MatMulSpecialized.from_csr(csr, 512, mapping_id=srt.named_mapping(4, "orig"), tile_config=same).get_config()
+    assert (real.b_staging, real.chunk_cols, real.nsplit) == (2, want.chunk_cols, want.nsplit)
