@@ -644,12 +644,14 @@ class Server:
         slot.launch(self.use_graphs)
         # Every result is copied out before the first block is given back, with
         # one wait for them all (one each took half the call at 24 requests).
-        with torch.cuda.stream(slot.stream):
+        try:
+            with torch.cuda.stream(slot.stream):
+                for r in batch:
+                    r.C = self.result_view(r).clone()
+        finally:  # a copy that fails (device memory) leaves no block behind
+            slot.stream.synchronize()
             for r in batch:
-                r.C = self.result_view(r).clone()
-        slot.stream.synchronize()
-        for r in batch:
-            self.release(r)
+                self.release(r)
 
     def serve(self, requests: List[Request], keep_results: bool = False) -> Dict[str, float]:
         """Open-loop serving of requests (arrival times in seconds from start).

@@ -157,3 +157,52 @@ def test_middle_widths_get_their_own_table(sv):
     for r in reqs:
         srv.release(r)
     assert srv.pool.used == 0 and srv.pool.live == 0
+
+
+def test_run_batch_gives_every_block_back_when_a_copy_fails(srt, monkeypatch):
+    """Results are copied out before the first block is given back; a copy that
+    fails leaves the budget as it was."""
+    import contextlib
+
+    import torch
+    sv = srt.serving
+    monkeypatch.setattr(torch.cuda, "stream", lambda s: contextlib.nullcontext())
+
+    class Stream:
+        def synchronize(self):
+            log.append("wait")
+
+    class Slot:
+        stream = Stream()
+
+        def launch(self, graphs):
+            log.append("launch")
+
+    class Result:
+        def __init__(self, ok):
+            self.ok = ok
+
+        def clone(self):
+            if not self.ok:
+                raise torch.OutOfMemoryError("no memory")
+            return "copy"
+
+    class Req:
+        def __init__(self, i):
+            self.i = i
+
+    for bad in (0, 2, None):
+        log, given = [], []
+        s = sv.Server.__new__(sv.Server)
+        s.slots, s.use_graphs = [Slot()], False
+        s.admit, s._fill = lambda r: True, lambda slot, batch: None
+        s.result_view = lambda r: Result(r.i != bad)
+        s.release = lambda r, *a, **kw: given.append((r.i, len(log)))
+        batch = [Req(i) for i in range(4)]
+        if bad is None:
+            s.run_batch(batch)
+            assert all(r.C == "copy" for r in batch)
+        else:
+            with pytest.raises(torch.OutOfMemoryError):
+                s.run_batch(batch)
+        assert given == [(i, 2) for i in range(4)] and log == ["launch", "wait"]
