@@ -68,3 +68,23 @@ def test_narrower_products_split_as_in_a_plan_of_their_own(srt, M, K, widths):
         plan(own, B)
         torch.cuda.synchronize()
         assert torch.equal(out, own)
+
+
+@pytest.mark.parametrize("mkn", [(64, 2048, 128), (129, 513, 129), (512, 2048, 256), (256, 4096, 512), (1024, 4096, 512),
+                                 (2064, 192, 1030), (33, 4000, 63)])
+def test_tile_and_split_change_no_bit(srt, mkn):
+    """A plan made for no columns has no workspace: every range of a tile in one
+    workgroup, and the tile that is fastest so.  The bits of the split launch."""
+    import torch
+    M, K, N = mkn
+    g = torch.Generator().manual_seed(M + K + N)
+    A = (torch.randn(M, K, generator=g) * (torch.rand(M, K, generator=g) < 0.5)).to_sparse_csr().cuda()
+    B = torch.randn(K, N, generator=g).cuda()
+    out = []
+    for n in (N, 0):
+        print("dense bits", mkn, n, flush=True)
+        plan = srt.MatMulSpecialized.from_csr(A, n, mapping_id=srt.named_mapping(4, "orig"), dense_threshold=0.2)
+        out.append(torch.full((M, N), float("nan"), device="cuda"))
+        plan(out[-1], B)
+    assert not bool(torch.isnan(out[0]).any())
+    assert torch.equal(out[0], out[1])

@@ -206,3 +206,48 @@ def test_open_plans_of_a_group_take_the_group_s_lane_width(srt, oracle):
                                  nsplit=p.split_counts())
             assert np.array_equal(C.cpu().numpy().view(np.uint32), ref.view(np.uint32))
         g.close()
+
+
+def test_operand_preparation_of_values_that_are_not_ordinary(srt):
+    """FP8 columns with NaN, infinities, signed zeros, and values so small that
+    their scale is subnormal or underflows to zero: the bytes of B / scale
+    rounded once to FP32, then NaN to 0x7f, saturated at +-448, nearest even."""
+    import torch
+    K, N = 200, 64
+    g = np.random.default_rng(8)
+    B = g.standard_normal((K, N)).astype(np.float32)
+    B[3, 0], B[5, 1], B[6, 2], B[7, 2], B[9, 3] = np.nan, np.inf, -np.inf, np.nan, -0.0
+    B[:, 4], B[:, 5] = -0.0, np.nan
+    B[:, 6] *= np.float32(1e-38)
+    B[:, 7] = (B[:, 7] * np.float32(1e-44)).astype(np.float32)
+    B[:, 8] *= np.float32(3e37)
+    B[1:, 9] *= np.float32(1e-7)  # one value at 448, the others far below the least subnormal
+    B[:, 10] = np.float32(448.0) * np.sign(B[:, 10])
+    mag = np.abs(B)
+    top = np.where(np.isnan(mag), 0, mag).max(axis=0)
+    with np.errstate(all="ignore"):
+        scale = np.where(top > 0, (top.astype(np.float64) / 448.0).astype(np.float32), np.float32(1))
+        q = (B.astype(np.float64) / scale.astype(np.float64)).astype(np.float32)
+    assert scale[7] == 0 and 0 < scale[6] < 2.0 ** -126 and np.isinf(scale[1])
+    ref = torch.from_numpy(np.clip(q, -448, 448)).to(torch.float8_e4m3fn).view(torch.uint8).numpy().copy()
+    ref[np.isnan(q)] = 0x7f
+    A = torch.zeros((16, K))
+    A[0, 0] = 1
+    Bq, t = srt.precision.PanelPlan.from_dense(A, "fp8").prepare_b(torch.from_numpy(B).cuda())
+    assert np.array_equal(t.cpu().numpy().view(np.uint32), scale.view(np.uint32))
+    assert np.array_equal(Bq.cpu().numpy()[:, :K].T, ref)
+
+
+@pytest.mark.parametrize("n_tile", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("N", [40, 100, 200])
+def test_csr_lane_width_is_the_columns_not_the_tile(srt, oracle, n_tile, N):
+    """One, two and four floats per lane (by N); n_tile changes no bit."""
+    import torch
+    _, cb = oracle
+    A = srt.workloads.magnitude_pruned(90, 300, 0.8, seed=N)
+    B = srt.workloads.dense_b(300, N, seed=N + 1)
+    rp, ci, v = srt.workloads.to_csr(A)
+    csr = torch.sparse_csr_tensor(torch.from_numpy(rp), torch.from_numpy(ci), torch.from_numpy(v), size=A.shape).cuda()
+    C = srt.csr.spmm(csr, torch.from_numpy(B).cuda(), n_tile=n_tile)
+    ref = cb.csr_exec(rp, ci, v, 90, B)
+    assert np.array_equal(C.cpu().numpy().view(np.uint32), ref.view(np.uint32))
