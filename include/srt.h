@@ -521,10 +521,11 @@ typedef struct srt_exec_problem {
  * whose operand fields the caller fills in later; then it must keep
  * b_bytes = K * ldb * 4 and the vec_width rules: vec_width | ldb, ldc; ldb
  * and ldc >= n rounded up to vec_width; 4 * vec_width-byte aligned B and C).
- * n need not be a multiple of vec_width: a lane's last vector reaches column
- * round_up(n, vec_width) - 1, so B's columns n .. that one are read (zeros
- * keep them harmless) and C's are overwritten; columns below n are the same
- * bits at every lane width. */
+ * n need not be a multiple of vec_width: the last lane moves back to columns
+ * n - vec_width .. n - 1, the same bits as the lane before it stores there.
+ * With n < vec_width a row's one vector covers vec_width columns: B's columns
+ * n .. vec_width - 1 are read (zeros keep them harmless) and C's overwritten.
+ * Columns below n are the same bits at every lane width. */
 int srt_exec_problem_fill(const srt_plan *p, const float *B, int64_t ldb, float *C, int64_t ldc, int n,
                           int vec_width, int block_begin, srt_exec_problem *out);
 int srt_exec_persistent_execute(const srt_plan *proto, int vec_width, const srt_exec_problem *d_probs,
@@ -541,8 +542,9 @@ int srt_exec_grouped_b_widen(const srt_bprep_problem *d_probs, const int *d_hdr,
 /* ------------------------------------------------------------------------
  * CSR baseline (sbench/SOP/_C/pytorch_csr_wrapper.cpp:243-312 _csr_kernel,
  * torch entry csr.executor :314-353): C[m x n] = A_csr * B, device arrays
- * rowptr[m+1], colind[nnz], vals[nnz].  n_tile in {16,32,64,128,256}
- * selects columns per wavefront (values below 64 run as 64); tails masked.
+ * rowptr[m+1], colind[nnz], vals[nnz].  n_tile in {16,32,64,128,256} is the
+ * reference's tile width, accepted and without effect: n selects the columns
+ * per wavefront (64, 128 above 64, 256 above 128); tails masked.
  * Row ranges are clamped to [0, nnz) and column indices outside [0, k) are
  * skipped, so malformed input cannot make the kernel read out of bounds.
  * ---------------------------------------------------------------------- */

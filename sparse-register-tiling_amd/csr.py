@@ -4,7 +4,8 @@
 reference's ``csr.executor`` (sbench/SOP/_C/pytorch_csr_wrapper.cpp:314-361):
 the CSR tensor's int32 or int64 indices are used as they are, the kernel is
 timed (median over blocks of ``num_runs`` runs) and C = A . B is returned.
-``spmm`` is the plain call.
+``spmm`` is the plain call.  ``n_tile`` (the reference's tile width) is
+accepted and checked; the kernel's columns per wavefront follow from B's.
 """
 from __future__ import annotations
 

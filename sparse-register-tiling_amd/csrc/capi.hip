@@ -2104,8 +2104,8 @@ int srt_exec_problem_fill(const srt_plan *p, const float *B, int64_t ldb, float 
         return fail(SRT_ERR_UNSUPPORTED, "the plan's schedule is not cut for unroll 4 (TileConfig.unroll = 4)");
     if (p->dense.ndense) return fail(SRT_ERR_UNSUPPORTED, "hybrid plans execute alone");
     if (n > 0 && (!B || !C)) return fail(SRT_ERR_INVALID, "null B or C");
-    // A lane's last vector reaches column round_up(n, V) - 1: the strides
-    // must hold it (B's columns there are read, C's are written).
+    // A row of fewer than V columns is one vector of V: the strides must hold it
+    // (B's columns there are read, C's are written), whatever n is later.
     const int64_t n_up = (int64_t)(n + V - 1) / V * V;
     if (ldb % V || ldc % V || ldb < n_up || ldc < n_up || !aligned(B, 4 * V) || !aligned(C, 4 * V))
         return fail(SRT_ERR_INVALID, "vec_width must divide ldb and ldc, both >= n rounded up to vec_width, and "
@@ -2470,8 +2470,8 @@ int srt_csr_spmm(int m, int k, int n, int64_t nnz, const void *rowptr, const voi
     if (ldb < n || ldc < n) return fail(SRT_ERR_INVALID, "ldb and ldc must be >= n");
     if (n_tile != 16 && n_tile != 32 && n_tile != 64 && n_tile != 128 && n_tile != 256)
         return fail(SRT_ERR_INVALID, "n_tile must be one of 16, 32, 64, 128, 256");
-    // n_tile is the reference's tile width; the same bits come out of every
-    // lane width, and the widest the columns fill reads B best.
+    // n_tile is the reference's tile width and changes nothing: the same bits come
+    // out of every lane width, and the widest the columns fill reads B best.
     const int V = n > 128 ? 4 : n > 64 ? 2 : 1;
     SRT_HIP_TRY(launch_csr(m, k, n, nnz, rowptr, colind, index_bytes, vals, B, ldb, C, ldc, V,
                            (hipStream_t)stream));

@@ -58,7 +58,7 @@ constexpr int kXcds = 8;
 constexpr int kMaxRanges = 32;
 constexpr int kMaxGroups = 8;
 
-// Workspace words (f32x4) of one (split, tile): every wave's accumulators.
+// Workspace words (f32x4) of one (group, tile): every wave's accumulators.
 constexpr int64_t tile_words(int tp, int nt16) { return (int64_t)tp * nt16 * 64; }
 
 template <bool kVecB, int kTP, int kNTiles>
@@ -93,7 +93,7 @@ __global__ void __launch_bounds__(kThreads)
     const __amdgpu_buffer_rsrc_t arsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<f32x4 *>(apack), (short)0, (int)a_bytes, 0x00020000);
 
-    // A staging: word e = tid + 512 r of the stage's [8 panels][4 groups][64 lanes]
+    // A staging: word e = tid + 512 r of the stage's [kTP panels][4 groups][64 lanes]
     f32x4 ra[kAW];
     fb rb[4];
     auto load_a = [&](int s, bool ok) {

@@ -42,11 +42,6 @@ struct VecOf<1> {
     typedef float type;
 };
 
-template <int V>
-__device__ __forceinline__ typename VecOf<V>::type load_vec(const float *p) {
-    return *reinterpret_cast<const typename VecOf<V>::type *>(p);
-}
-
 // V floats at a 4-byte aligned address: one wide memory instruction as well
 // (global and buffer accesses of this chip need dword alignment only).
 template <int V>
