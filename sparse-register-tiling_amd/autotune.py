@@ -506,13 +506,17 @@ def hybrid_choices(csr: torch.Tensor, N: int, plan: MatMulSpecialized, path: str
     as the whole matrix has it.  Neither leads: 1956 x 1351 at 69 % x 177, 70 of
     123 panels dense, takes 43.7 us with the first and 33.7 with the second, 792
     x 1275 at 68 % x 249, 2 of 50, 23.5 and 30.0.  Where the plan streams, the
-    default alone, since the few rows a hybrid leaves would stream all of B
-    (4096 x 1024 x 512: 71.9 us with 3 of 256 panels left to streaming, 55.9
-    with 7 left to the gather)."""
+    default mapping: the few rows a hybrid leaves would stream all of B (4096 x
+    1024 x 512: 71.9 us with 3 of 256 panels left to streaming, 55.9 with 7 left
+    to the gather)."""
     mapping, cfg = plan_choice(csr, N, path)
-    if cfg is not None and cfg.b_staging == 3:
-        return named_mapping(4, "orig"), [None]
-    return mapping, [cfg, plan.get_config()]
+    if cfg is None or cfg.b_staging != 3:
+        return mapping, [cfg, plan.get_config()]
+    mapping = named_mapping(4, "orig")
+    whole = MatMulSpecialized.from_csr(csr, N, mapping_id=mapping)
+    configs = [None, whole.get_config()]
+    whole.close()
+    return mapping, configs
 
 
 HYBRID_THRESHOLDS = (0.2, 0.25, 0.3, 0.35, 0.4)

@@ -205,3 +205,16 @@ def test_tuned_hybrids_also_try_the_launch_for_the_panels_that_are_left(srt, mon
     plan(C, B)
     Ad = A.to_dense().cuda().double()
     assert bool(((C.double() - Ad @ B.double()).abs() <= (Ad @ B.double()) * (K + 40) * 2.0 ** -24).all())
+
+
+def test_hybrids_of_a_streamed_plan_gather(srt):
+    """Where the tuned plan streams, the rows beside the dense panels are timed
+    on the 4-row default, for themselves and as the whole matrix would have it."""
+    import torch
+    g = torch.Generator().manual_seed(4)
+    A = (torch.rand((4096, 1000), generator=g) < 0.3).float().to_sparse_csr()
+    plan = srt.autotune.tuned_plan(A, 520)
+    assert plan.get_config().b_staging == 3
+    mapping, configs = srt.autotune.hybrid_choices(A, 520, plan)
+    whole = srt.MatMulSpecialized.from_csr(A, 520, mapping_id=srt.named_mapping(4, "orig")).get_config()
+    assert mapping.M_r == 4 and configs == [None, whole] and whole.b_staging == 2
