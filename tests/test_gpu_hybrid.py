@@ -213,8 +213,8 @@ def test_hybrids_of_a_streamed_plan_gather(srt):
     import torch
     g = torch.Generator().manual_seed(4)
     A = (torch.rand((4096, 1000), generator=g) < 0.3).float().to_sparse_csr()
-    plan = srt.autotune.tuned_plan(A, 520)
+    plan = srt.autotune.tuned_plan(A, 640)
     assert plan.get_config().b_staging == 3
-    mapping, configs = srt.autotune.hybrid_choices(A, 520, plan)
-    whole = srt.MatMulSpecialized.from_csr(A, 520, mapping_id=srt.named_mapping(4, "orig")).get_config()
+    mapping, configs = srt.autotune.hybrid_choices(A, 640, plan)
+    whole = srt.MatMulSpecialized.from_csr(A, 640, mapping_id=srt.named_mapping(4, "orig")).get_config()
     assert mapping.M_r == 4 and configs == [None, whole] and whole.b_staging == 2
