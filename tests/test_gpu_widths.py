@@ -251,3 +251,71 @@ def test_csr_lane_width_is_the_columns_not_the_tile(srt, oracle, n_tile, N):
     C = srt.csr.spmm(csr, torch.from_numpy(B).cuda(), n_tile=n_tile)
     ref = cb.csr_exec(rp, ci, v, 90, B)
     assert np.array_equal(C.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("index_dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("N", [65, 127, 128, 129, 255, 258, 515])
+def test_csr_many_short_rows(srt, oracle, index_dtype, N):
+    """Enough rows of few entries for the short-row kernel, rows of every length
+    around its batches, its long rows and their batches among them, the last
+    workgroup short of rows; columns in no order and outside the matrix."""
+    import torch
+    _, cb = oracle
+    rng = np.random.default_rng(N)
+    M, K = 4099, 300
+    lengths = rng.integers(0, 6, M)
+    edges = [0, 1, 3, 4, 5, 7, 8, 9, 31, 32, 33, 34, 47, 48, 49, 63, 64, 65, 80, 81, 96, 97, 127, 128, 129, 200, 300]
+    lengths[rng.permutation(M)[:len(edges)]] = edges
+    lengths[-3:] = [33, 2, 70]
+    lengths[8:12] = [64, 65, 40, 300]  # a workgroup of long rows
+    rp = np.concatenate([[0], np.cumsum(lengths)]).astype(index_dtype)
+    assert rp[-1] <= 8 * M
+    ci = np.concatenate([rng.permutation(K)[:l] for l in lengths]).astype(index_dtype)
+    v = rng.standard_normal(len(ci)).astype(np.float32)
+    B = rng.uniform(-1, 1, (K, N)).astype(np.float32)
+    ref = cb.csr_exec(rp.astype(np.int64), ci.astype(np.int64), v, M, B)
+    wide = torch.full((K, N + 5), float("nan"), device="cuda")
+    wide[:, 3:3 + N] = torch.from_numpy(B).cuda()
+    parts = tuple(torch.from_numpy(x).cuda() for x in (rp, ci, v))
+    A = torch.sparse_csr_tensor(torch.zeros(M + 1, dtype=torch.int64), torch.zeros(0, dtype=torch.int64), torch.zeros(0),
+                                size=(M, K))
+    C = torch.full((M, N + 3), 7.0, device="cuda")
+    srt.csr.spmm(A, wide[:, 3:3 + N], C[:, 1:1 + N], _parts_cache=parts)
+    torch.cuda.synchronize()
+    got = C.cpu().numpy()
+    assert np.array_equal(np.ascontiguousarray(got[:, 1:1 + N]).view(np.uint32), ref.view(np.uint32))
+    assert (got[:, 0] == 7.0).all() and (got[:, 1 + N:] == 7.0).all()
+    # entries outside the matrix are left out: the product without them
+    out = rng.random(len(ci)) < 0.1
+    bad = ci.copy()
+    bad[out] = rng.choice([-1, K, K + 7, -1000], int(out.sum())).astype(index_dtype)
+    keep = np.concatenate([[0], np.cumsum(~out)])
+    ref = cb.csr_exec(keep[rp].astype(np.int64), ci[~out].astype(np.int64), v[~out], M, B)
+    got = srt.csr.spmm(A, torch.from_numpy(B).cuda(), _parts_cache=(parts[0], torch.from_numpy(bad).cuda(), parts[2]))
+    assert np.array_equal(got.cpu().numpy(), ref)
+
+
+def test_csr_short_rows_with_row_pointers_out_of_order(srt):
+    """Row pointers that fall or leave [0, nnz]: clamped, as by the other kernel
+    (the same rows with enough entries behind them that it takes them)."""
+    import torch
+    M, K, N, nnz = 4099, 200, 130, 20000
+    g = torch.Generator().manual_seed(3)
+    rp = torch.sort(torch.randint(0, nnz, (M + 1,), generator=g)).values
+    rp[5], rp[100], rp[200], rp[4000], rp[-1] = -7, 3, nnz + 9, 0, nnz + 100
+    ci = torch.randint(0, K, (16 * M,), generator=g)
+    v = torch.randn(16 * M, generator=g)
+    B = torch.rand((K, N), generator=g).cuda()
+    A = torch.sparse_csr_tensor(torch.zeros(M + 1, dtype=torch.int64), torch.zeros(0, dtype=torch.int64), torch.zeros(0),
+                                size=(M, K))
+    short = srt.csr.spmm(A, B, _parts_cache=(rp.cuda(), ci[:nnz].cuda(), v[:nnz].cuda()))
+    # the same ranges, written out, in arrays of 16 entries a row
+    lo = rp[:-1].clamp(0, nnz)
+    fixed = torch.stack([lo, torch.maximum(rp[1:].clamp(max=nnz), lo)])
+    lengths = fixed[1] - fixed[0]
+    at = torch.cat([torch.arange(int(a), int(b)) for a, b in zip(fixed[0].tolist(), fixed[1].tolist())])
+    ptr = torch.cat([torch.zeros(1, dtype=torch.int64), torch.cumsum(lengths, 0)])
+    pad = 9 * M
+    long = srt.csr.spmm(A, B, _parts_cache=(ptr.cuda(), torch.cat([ci[at], ci[:pad]]).cuda(),
+                                            torch.cat([v[at], v[:pad]]).cuda()))
+    assert torch.equal(short, long)
