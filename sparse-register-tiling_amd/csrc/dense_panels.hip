@@ -29,9 +29,10 @@
 // stages ahead gave no more (156 us against 154 at 1024 x 16384 x 512): large
 // products run at 0.76 of the matrix cores' cycles.
 //
-// K is cut into ranges, one chain of additions each, and ranges into at most
-// eight groups; a range's sum joins its group's, the groups' sums are added in
-// order.  A workgroup takes whole groups, so tile and split change no bit of C.
+// K is cut into ranges, one chain of additions each, and ranges into groups (long
+// ones each its own, short ones at most eight); a range's sum joins its group's,
+// the groups' sums are added in order.  A workgroup takes whole groups, so tile
+// and split change no bit of C.
 // With S > 1 workgroups per tile each stores its groups' sums (lane order) to a
 // workspace, and dense_tiles_reduce adds them in order and writes C: results
 // repeat bit for bit.
@@ -56,7 +57,7 @@ constexpr int kWaves = 8;
 constexpr int kThreads = 64 * kWaves;
 constexpr int kXcds = 8;
 constexpr int kMaxRanges = 32;
-constexpr int kMaxGroups = 8;
+constexpr int kFewGroups = 8;
 
 // Workspace words (f32x4) of one (group, tile): every wave's accumulators.
 constexpr int64_t tile_words(int tp, int nt16) { return (int64_t)tp * nt16 * 64; }
@@ -312,8 +313,8 @@ __global__ void __launch_bounds__(256)
 }
 
 // Tile and K split of a launch.  K is cut into the ranges that fill the chip
-// with 128 x 128 tiles, at most 32 (SPC stages each); CPG ranges form a group,
-// at most 8 groups; a workgroup takes GPS groups.
+// with 128 x 128 tiles, at most 32 (SPC stages each); CPG ranges form a group; a
+// workgroup takes GPS of the Q groups.
 struct DenseGrid {
     int tp, nt16, PT, NT, SPC, CPG, Q, GPS, S;
 };
@@ -330,7 +331,7 @@ int dense_ranges(int ndense, int stages, int N, int *stages_each) {
 // to gain 6 %.  The model, in us: a launch, a stage of a workgroup's chain, the
 // matrix work of the CU with most workgroups, the operand bytes, and for a
 // split the second launch and its partials.  Least squares over 123 problems
-// (256..4096 rows and depth, 32..2048 columns); its choice takes 1.015 of the
+// (256..4096 rows and depth, 32..2048 columns); its choice takes 1.02 of the
 // fastest launch's time on average, 128 x 128 tiles with a workgroup per range,
 // the only launch before, 1.35 (512 x 512 x 128: 12.0 us, now 6.8; 512 x 2048 x
 // 256: 21.3, now 13.5; 4096 x 4096 x 64: 47.0, now 28.8; 2048 x 2048 x 1024: 83
@@ -343,7 +344,11 @@ DenseGrid dense_grid(int ndense, int G, int N, size_t ws_words) {
     const int stages = std::max(1, (G + kSG - 1) / kSG);
     DenseGrid best{}, g;
     const int ranges = dense_ranges(ndense, stages, N, &g.SPC);
-    g.CPG = (ranges + kMaxGroups - 1) / kMaxGroups;
+    // A range of three stages or more is its own group, which keeps 128 x 128
+    // tiles busy; shorter ones form at most eight, since their partials would
+    // cost more (2920 x 2692 x 128, 11 ranges of 4 stages: 36.8 us in 6 groups,
+    // 30.1 in 11; 761 x 1012 x 192, 16 of 1: 13.0 in 8, 16.9 in 16).
+    g.CPG = g.SPC >= 3 ? 1 : (ranges + kFewGroups - 1) / kFewGroups;
     g.Q = (ranges + g.CPG - 1) / g.CPG;
     double best_t = -1.0;
     for (const auto &tile : kTiles) {

@@ -88,3 +88,23 @@ def test_tile_and_split_change_no_bit(srt, mkn):
         plan(out[-1], B)
     assert not bool(torch.isnan(out[0]).any())
     assert torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("mkn", [(33, 8192, 63), (1500, 2692, 127), (1500, 1472, 128), (16, 6100, 300)])
+def test_long_ranges_are_their_own_groups(srt, mkn):
+    """More than eight groups of three stages and more; the third has shorter ones, in eight groups."""
+    import torch
+    M, K, N = mkn
+    g = torch.Generator().manual_seed(M + K + N)
+    A = torch.randn(M, K, generator=g) * (torch.rand(M, K, generator=g) < 0.5)
+    B = torch.randn(K, N, generator=g).cuda()
+    ref, mag = A.double() @ B.cpu().double(), A.abs().double() @ B.cpu().abs().double()
+    out = []
+    for n in (N, 0):
+        print("dense groups", mkn, n, flush=True)
+        plan = srt.MatMulSpecialized.from_csr(A.to_sparse_csr().cuda(), n, mapping_id=srt.named_mapping(4, "orig"),
+                                              dense_threshold=0.2)
+        out.append(torch.full((M, N), float("nan"), device="cuda"))
+        plan(out[-1], B)
+    assert bool(((out[0].cpu().double() - ref).abs() <= K * 2.0 ** -24 * mag + 1e-30).all())
+    assert torch.equal(out[0], out[1])
