@@ -205,6 +205,17 @@ __global__ void __launch_bounds__(1024)
     }
 }
 
+// The same where rows are few: a thread per column, 256 columns a block.
+__global__ void __launch_bounds__(256)
+    col_scale_few_kernel(int rows, int cols, const float *__restrict__ src, int64_t ld, float *__restrict__ scale) {
+    const int c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= cols) return;
+    float m = 0.0f;
+#pragma unroll 4
+    for (int r = 0; r < rows; ++r) m = fmaxf(m, fabsf(src[r * ld + c]));
+    scale[c] = m > 0.0f ? (float)((double)m / 448.0) : 1.0f;
+}
+
 // fp32 B (K x N, row-major) -> Bt (N x ldk, k contiguous) in BF16 or e4m3,
 // k in [K, ldk) zero: the MFMA B operand wants eight consecutive k of one
 // column per lane.  A tile of 32 columns and one 128-byte line of k per output
@@ -632,8 +643,18 @@ hipError_t launch_b_convert(int64_t rows, int cols, const float *src, int64_t ld
     const dim3 grid((unsigned)((ldk + tk - 1) / tk), (unsigned)((cols + 31) / 32));
     const int wide = (uintptr_t)dst % 16 == 0 && ldk * esz % 16 == 0;
     if (fp8) {
-        hipLaunchKernelGGL(col_scale_kernel, dim3((cols + 15) / 16), dim3(1024), 0, s, rows, cols, src, ld_src,
-                           cscale);
+        // With few rows most of a block of 1024 threads idles, and over many
+        // columns there are many such blocks; with more rows a thread's walk is
+        // the longer one.  us for blocks of 16 columns / a thread per column:
+        // 32 x 2000 6.3 / 6.1, 32 x 60000 20.6 / 9.6, 64 x 2000 6.3 / 7.0,
+        // 64 x 10000 8.2 / 7.4, 128 x 10000 9.0 / 9.4, 256 x 60000 43.9 / 38.3,
+        // 512 x 60000 65.0 / 69.5.
+        if (rows <= 32 || (rows <= 256 && rows * 100 <= cols))
+            hipLaunchKernelGGL(col_scale_few_kernel, dim3((cols + 255) / 256), dim3(256), 0, s, (int)rows, cols, src,
+                               ld_src, cscale);
+        else
+            hipLaunchKernelGGL(col_scale_kernel, dim3((cols + 15) / 16), dim3(1024), 0, s, rows, cols, src, ld_src,
+                               cscale);
         hipLaunchKernelGGL(b_transpose_kernel<true>, grid, dim3(256), 0, s, (int)rows, cols, src, ld_src, cscale,
                            (uint8_t *)dst, ldk, wide);
     } else {

@@ -319,3 +319,26 @@ def test_csr_short_rows_with_row_pointers_out_of_order(srt):
     long = srt.csr.spmm(A, B, _parts_cache=(ptr.cuda(), torch.cat([ci[at], ci[:pad]]).cuda(),
                                             torch.cat([v[at], v[:pad]]).cuda()))
     assert torch.equal(short, long)
+
+
+@pytest.mark.parametrize("K,N", [(1, 1), (1, 255), (32, 257), (33, 3299), (33, 3300), (64, 6400), (256, 25601), (257, 25700)])
+def test_fp8_scales_of_few_rows(srt, K, N):
+    """Both kernels of the column scales, around the lines between them: the
+    exact scale of every column of a view with rows 4-byte aligned, zero, NaN
+    and infinite columns among them."""
+    import torch
+    print("fp8 scales of few rows", K, N, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(K + N)
+    B = torch.full((K, N + 5), float("nan"), device="cuda")[:, 3:3 + N]
+    B.copy_(torch.randn((K, N), generator=g, device="cuda") * torch.exp(4 * torch.randn((1, N), generator=g, device="cuda")))
+    if N > 8:
+        B[:, 3] = 0
+        B[K // 2, 4] = float("nan")
+        B[K - 1, 5] = float("-inf")
+        B[:, 6] = -0.0
+    A = torch.zeros((16, K))
+    A[0, 0] = 1
+    _, t = srt.precision.PanelPlan.from_dense(A, "fp8").prepare_b(B)
+    top = torch.where(B.isnan(), torch.zeros_like(B), B.abs()).amax(dim=0).double()
+    scale = torch.where(top > 0, (top / 448.0).float(), torch.ones_like(t))
+    assert torch.equal(t.view(torch.int32), scale.view(torch.int32))
