@@ -40,13 +40,15 @@ def _index_tensor(x, device) -> torch.Tensor:
 
 
 # Time model of default_launch, in us: (a launch; a K block of one
-# workgroup's chain, by shape; 10 KB of operand tiles per CU; the second launch of
-# a K split; a million floats of partial tiles).  Least squares over 66 problem
+# workgroup's chain, by shape; 10 KB of operand tiles of the CU with most
+# workgroups; the second launch of a K split; a million floats of partial tiles).  Least squares over 66 problem
 # sizes (256..4096 rows, 128..4096 deep, 32..2048 columns) times the three shapes
 # times K splits of 1..32.  On average its choice takes 1.03 of the fastest
 # launch's time; 64-column tiles with the K range split up to 256 workgroups,
 # which it replaces, took 1.23 (512 x 512 x 100: 8.1 us, now 6.7; 2048 x 512 x
-# 512: 14.2, now 7.9; 4096 x 1024 x 1024: 19.7 both).
+# 512: 14.2, now 7.9; 4096 x 1024 x 1024: 19.7 both).  Workgroups past a full
+# chip count as a round of their own: 240 x 6214 x 4258 takes 54.0 us in 134
+# workgroups of 64 columns, 60.0 in 268 of 32.
 _LAUNCH_US = 5.39
 _CHAIN_US = ((6, .151), (9, .103), (4, .091))
 _TILE_US, _SPLIT_US, _PARTIAL_US = .101, 1.49, 1.52
@@ -77,8 +79,9 @@ def default_launch(num_panels: int, k_blocks: int, n: int, target_groups: int = 
         ks = 1
         while ks <= limit:
             steps = -(-k_blocks // ks)
-            t = _LAUNCH_US + chain * steps
-            t += _TILE_US * groups * ks * steps * (wp * pw * 1024 + nt * 64) / target_groups * 1e-4
+            rounds = groups * ks / target_groups
+            rounds = -(-groups * ks // target_groups) if rounds > 1 else rounds
+            t = _LAUNCH_US + chain * steps + _TILE_US * rounds * steps * (wp * pw * 1024 + nt * 64) * 1e-4
             if ks > 1:
                 t += _SPLIT_US + _PARTIAL_US * (ks + 1) * num_panels * 16 * n * 1e-6
             if best is None or t < best[0]:

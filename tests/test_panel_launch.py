@@ -25,6 +25,16 @@ def test_rule_stays_within_its_workspace(pr):
                 assert ks == 1 or ks * 4 <= blocks
 
 
+@pytest.mark.parametrize("m,k,n", [(228, 4203, 4622), (240, 6214, 4258), (1024, 4096, 1024)])
+def test_wide_products_stay_in_one_round(pr, m, k, n):
+    """64-column tiles that nearly fill the chip are not cut into 32-column ones
+    of which a few run after all others."""
+    panels, blocks = -(-m // 16), -(-k // 32)
+    shape, ks = pr.default_launch(panels, blocks, n)
+    nt, wp, pw = pr.SHAPES[shape]
+    assert -(-panels // (wp * pw)) * -(-n // nt) * ks <= 256
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["bf16", "fp8"])
 @pytest.mark.parametrize("ks", [2, 3, 4, 5, 6, 9])
