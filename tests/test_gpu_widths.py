@@ -342,3 +342,26 @@ def test_fp8_scales_of_few_rows(srt, K, N):
     top = torch.where(B.isnan(), torch.zeros_like(B), B.abs()).amax(dim=0).double()
     scale = torch.where(top > 0, (top / 448.0).float(), torch.ones_like(t))
     assert torch.equal(t.view(torch.int32), scale.view(torch.int32))
+
+
+@pytest.mark.parametrize("K,N,ld", [(748, 11215, 11215), (640, 13120, 13121), (1100, 7627, 7630)])
+def test_prepared_b_of_many_unaligned_rows(srt, K, N, ld):
+    """Tiles of k that 8 does not divide, and rows that start inside a line."""
+    import torch
+    print("prepared B, unaligned rows", K, N, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(K + N)
+    B = torch.full((K, ld), float("nan"), device="cuda")[:, ld - N:]
+    B.copy_(torch.randn((K, N), generator=g, device="cuda"))
+    ldk = -(-K // 32) * 32
+    A = torch.zeros((16, K))
+    A[0, 0] = 1
+    Bt, _ = srt.precision.PanelPlan.from_dense(A, "bf16").prepare_b(B)
+    ref = torch.zeros((N, ldk), dtype=torch.bfloat16, device="cuda")
+    ref[:, :K] = B.t().to(torch.bfloat16)
+    assert torch.equal(Bt.view(torch.int16), ref.view(torch.int16))
+    Bq, t = srt.precision.PanelPlan.from_dense(A, "fp8").prepare_b(B)
+    scale = (B.abs().amax(dim=0).double() / 448.0).float()
+    assert torch.equal(t, scale)
+    q = torch.zeros((N, ldk), dtype=torch.uint8, device="cuda")
+    q[:, :K] = (B.double() / scale.double()).float().t().contiguous().to(torch.float8_e4m3fn).view(torch.uint8)
+    assert torch.equal(Bq, q)
