@@ -171,6 +171,19 @@ def test_default_lane_width(srt, M, K, s, N, V):
     assert plan.get_config().vec_width == V
 
 
+@pytest.mark.parametrize("M,K,s,N,halved", [(64, 6325, 0.928, 2605, False), (260, 2497, 0.975, 3110, True),
+                                            (3492, 7320, 0.991, 309, True), (1024, 4096, 0.9, 128, False)])
+def test_default_chunk_is_halved_where_a_panel_has_few(srt, M, K, s, N, halved):
+    """More than four N tiles and fewer than four chunks a panel: half the columns a chunk."""
+    import torch
+    csr = (torch.rand(M, K, device="cuda") >= s).float().to_sparse_csr()
+    plan = srt.MatMulSpecialized.from_csr(csr, N, mapping_id=srt.named_mapping(4, "orig"),
+                                          tile_config=srt.TileConfig(vec_width=1))
+    whole = -(-plan.stats()["packed_cols"] * -(-N // 64) // 4096)
+    assert whole > 60
+    assert plan.get_config().chunk_cols == (max(60, whole // 2) if halved else whole)
+
+
 def test_open_plans_of_a_group_take_the_group_s_lane_width(srt, oracle):
     """Plans that leave the lane width open: a lone launch of these has too few
     workgroups for wide lanes, the group has not.  One problem of few columns
