@@ -605,18 +605,22 @@ static int cu_count() {
 // "orig", us at 4 / 2 / 1: 1211 x 9904 at 89 % x 199 164 / 132 / 109, 2699 x
 // 6439 at 98.5 % x 104 45 / 41 / 25, 4163 x 2281 at 92 % x 384 62 / 98 / 101,
 // 2424 x 524 at 71 % x 320 25 / 39 / 27.  Few rows of B under many columns are
-// bound by the stores of C: 63 x 199 at 58 % x 3168 5.9 / 7.5 / 8.0.  Over 350
-// drawn sizes (16..10000 rows, 16..12000 deep, 16..8192 columns, 50..99.7 %) it
-// takes 1.017 of the fastest width's time on average, the widest lane that
-// gives a workgroup per CU 1.038 and up to 1.67 times it.
+// bound by the stores of C (63 x 199 at 58 % x 3168 5.9 / 7.5 / 8.0) and little
+// work by its launch (2365 x 169 at 99.6 % x 516, 8-row, 5.9 / - / 7.0), unless
+// the workgroups do not fill the chip (42 x 70 at 88 % x 2373, 8-row, 6.2 / 5.5
+// / 5.4).  Up to 128 columns two floats want 50 gathers of a row: 5334 x 4719 at
+// 99.5 % x 88, 26 of them, - / 22.6 / 14.5.  Over 1400 drawn sizes (16..10000
+// rows, 16..12000 deep, 16..8192 columns, 50..99.7 %) lanes and chunks take
+// 1.025 of the fastest time on average.
 //   slices, wide: panels x 64- and x 256-column slices of the whole launch.
 static int default_lanes(int64_t slices, int64_t wide, int K, int64_t total_cols, int n) {
     const int64_t cus = cu_count();
     const int64_t per_xcd = std::min<int64_t>(8, (n + 255) / 256);  // eighths of the gathers that one XCD makes
     if (n > 128 && (slices > 12 * cus || (total_cols * per_xcd >= 8 * 16 * (int64_t)K && 2 * wide >= cus) ||
-                    (K <= 256 && n >= 1024)))
+                    (K <= 256 && n >= 1024 && 4 * wide >= 3 * cus) ||
+                    (total_cols * ((n + 63) / 64) <= 8 * 4096 && 2 * wide >= 3 * cus)))
         return 4;
-    return n > 64 && slices > 10 * cus ? 2 : 1;
+    return n > 64 && slices > 10 * cus && total_cols >= 50 * (int64_t)K ? 2 : 1;
 }
 
 // Realise the GPU fields of a tile config for a matrix of K columns with

@@ -184,6 +184,17 @@ def test_default_chunk_is_halved_where_a_panel_has_few(srt, M, K, s, N, halved):
     assert plan.get_config().chunk_cols == (max(60, whole // 2) if halved else whole)
 
 
+@pytest.mark.parametrize("M,K,s,N,V", [(5334, 4719, 0.9951, 88, 1), (6034, 3033, 0.9944, 80, 1), (3002, 3357, 0.9869, 201, 1),
+                                       (5200, 1892, 0.924, 128, 2), (42, 70, 0.8787, 2373, 1), (192, 238, 0.9896, 3020, 4),
+                                       (3122, 165, 0.9911, 152, 4), (166, 529, 0.9957, 4028, 4), (331, 10472, 0.9293, 983, 1)])
+def test_default_lane_width_with_few_gathers(srt, M, K, s, N, V):
+    """Rows of B that few panels gather are read by narrow lanes, unless the whole work is small."""
+    import torch
+    csr = (torch.rand(M, K, device="cuda") >= s).float().to_sparse_csr()
+    plan = srt.MatMulSpecialized.from_csr(csr, N, mapping_id=srt.named_mapping(4, "orig"))
+    assert plan.get_config().vec_width == V
+
+
 def test_open_plans_of_a_group_take_the_group_s_lane_width(srt, oracle):
     """Plans that leave the lane width open: a lone launch of these has too few
     workgroups for wide lanes, the group has not.  One problem of few columns
