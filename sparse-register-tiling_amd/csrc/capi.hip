@@ -631,11 +631,12 @@ static int default_lanes(int64_t slices, int64_t wide, int K, int64_t total_cols
 // Waves: 8 at every size (plans of one group have to agree).  16 are about a
 // twentieth faster on small products and up to a half slower on large ones
 // (996 x 2291 x 2344, 4-row "orig": 1.29 of the time of 8).  Chunks: with more
-// than four N tiles and fewer than four chunks a panel, workgroups are many, and
-// half as many columns a chunk even out the CUs: 0.90 of the time on average
-// over 825 launches (0.29 to 1.35); with fewer tiles (1.03 over 491) or more
-// chunks (1.00 over 250, up to 1.36: 64 x 6325 at 93 % x 2605 52.5 us, 67.1 so)
-// the extra ones only open a second round.
+// than four N tiles workgroups are many, and half as many columns a chunk even
+// out the CUs: 0.90 of the time on average over 825 launches with fewer than
+// four chunks a panel (0.29 to 1.35), 0.98 over 125 with more where a row of B
+// is gathered 12 times.  Else (1.02 over 125) and with fewer tiles (1.03 over
+// 491) the extra chunks only open a second round (64 x 6325 at 93 % x 2605 52.5
+// us, 67.1 so).
 static void realise_config(srt_tile_config &c, int P, int M_r, int K, int K_tile, int64_t total_cols, int n) {
     if (c.b_staging == 3) c.chunk_cols = c.nsplit = 0;  // a streamed plan's, C rows per wave: nothing of this executor
     if (c.vec_width != 1 && c.vec_width != 2 && c.vec_width != 4)
@@ -662,7 +663,8 @@ static void realise_config(srt_tile_config &c, int P, int M_r, int K, int K_tile
         const int64_t n_tiles = (n + 64 * c.vec_width - 1) / (64 * c.vec_width);
         const int64_t target_waves = 4096;
         c.chunk_cols = (int)std::max<int64_t>(8, (total_cols * n_tiles + target_waves - 1) / target_waves);
-        if (own && n_tiles > 4 && c.chunk_cols > 60 && total_cols < 4 * (int64_t)P * c.chunk_cols)
+        if (own && n_tiles > 4 && c.chunk_cols > 60 &&
+            (total_cols < 4 * (int64_t)P * c.chunk_cols || total_cols >= 12 * (int64_t)K))
             c.chunk_cols = std::max(60, c.chunk_cols / 2);
     }
     if (c.xcd_remap != 0 && c.xcd_remap != 1) c.xcd_remap = 1;

@@ -171,7 +171,7 @@ def test_default_lane_width(srt, M, K, s, N, V):
     assert plan.get_config().vec_width == V
 
 
-@pytest.mark.parametrize("M,K,s,N,halved", [(64, 6325, 0.928, 2605, False), (260, 2497, 0.975, 3110, True),
+@pytest.mark.parametrize("M,K,s,N,halved", [(64, 6325, 0.928, 2605, False), (260, 2497, 0.975, 3110, True), (148, 2003, 0.54, 1564, True),
                                             (3492, 7320, 0.991, 309, True), (1024, 4096, 0.9, 128, False)])
 def test_default_chunk_is_halved_where_a_panel_has_few(srt, M, K, s, N, halved):
     """More than four N tiles and fewer than four chunks a panel: half the columns a chunk."""
